@@ -215,10 +215,11 @@ typedef struct mjhOption {
 /* ---- data ---- */
 /* step_desc: optional device buffer of MJH_STEP_DESC_WORDS words (ndesc)
  * that mjh_step_fused (and, for nv <= 32, mjh_solve and so mjh_step) fills
- * with the model / data description each call (by a one-thread kernel, so
- * the call stays capturable) and whose kernels then read it from device
- * memory; a model passed only as a kernel argument compiles to slower code
- * for these kernels (part of it copied to scratch memory, more registers).
+ * with the model / data description each call (by a small kernel, so the
+ * call stays capturable) and whose kernels then read it from device memory;
+ * a model passed only as a kernel argument compiles to slower code for these
+ * kernels (part of it copied to scratch memory, more registers).  The second
+ * half holds a bit per world for the big-world launch (see world_flags).
  * NULL: the kernel-argument path, with the same results. */
 #define MJH_STEP_DESC_WORDS 2048
 

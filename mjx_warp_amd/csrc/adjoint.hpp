@@ -209,7 +209,8 @@ MJH_DEV void adjoint_vjp(const mjhModel& m, const mjhData& d, const float* qpos_
   const float* a_i = advances_with_qacc(m) ? a_s : WPTR(d.qacc_integration, w, nv);
   const bool damp = !advances_with_qacc(m) && (m.opt.integrator == mjhINT_EULER || passive_on);
 
-  float* cv = lds;
+  float* cbuf = lds + (t.lane & 32);  // first: read as float4s
+  float* cv = lds + 64;
   float* caA = cv + 6 * nb;
   float* caS = caA + 6 * nb;
   float* Vm = caS + 6 * nb;
@@ -229,7 +230,7 @@ MJH_DEV void adjoint_vjp(const mjhModel& m, const mjhData& d, const float* qpos_
   float* tmp = wv + nv;
   int* blk = (int*)(tmp + nv);
   float* A = (float*)(blk + nv);
-  float* rlf = A + nv * nv + 64;
+  float* rlf = A + nv * nv;
   float* rg = rlf + rcap;
   float* rcq = rg + rcap;
   float* rcv = rcq + rcap;
@@ -289,7 +290,6 @@ MJH_DEV void adjoint_vjp(const mjhModel& m, const mjhData& d, const float* qpos_
   // larger: the LDS factor
   const bool reg = nv <= kRegNvMax;
   const int rl = t.lane & 31;
-  float* cbuf = A + nv * nv + (t.lane & 32);
   int rbeg = rl, rend = rl + 1;
   if (reg && rl < nv) tree_block(m, rl, &rbeg, &rend);
   if (reg) {
@@ -298,7 +298,7 @@ MJH_DEV void adjoint_vjp(const mjhModel& m, const mjhData& d, const float* qpos_
     const float x = with_nvc(nv, [&](auto nvc) {
       RegChol<decltype(nvc)::value> c{rl, cbuf};
       c.load_sym(qM, nv, rbeg, rend, dg);
-      c.factor();
+      c.template factor<false>();
       return c.solve(b);
     });
     if (t.lane < nv) mu[t.lane] = x;
@@ -363,7 +363,7 @@ MJH_DEV void adjoint_vjp(const mjhModel& m, const mjhData& d, const float* qpos_
         for (int j = 0; j < NVC; j++)
           if (j < nv) c.h[j] = fmaf(g, Ji[j], c.h[j]);
       }
-      c.factor();
+      c.template factor<false>(true);
       return c.solve(b);
     });
     sync();

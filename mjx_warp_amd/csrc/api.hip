@@ -39,9 +39,7 @@ int fail(int code, const std::string& msg) {
   return code;
 }
 __global__ void k_reset(mjhData d, int which) {
-  if (threadIdx.x == 0) {
-    reset_counters(d, which);
-  }
+  reset_counters(d, which);
 }
 
 // res = M vec / x = inv(M) y / qfrc += J' xfrc for caller-provided vectors
@@ -83,6 +81,7 @@ MJH_DEV int pool_rows(const mjhData& d) { return min(max(d.nefc[0], 0), d.njmax)
 
 // per world: clear the block and the counter bits (keeps the flags)
 __global__ void k_blocks_zero(mjhData d) {
+  if (blockIdx.x == 0) clear_big_map(d, threadIdx.x, blockDim.x);
   for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < d.nworld; w += gridDim.x * blockDim.x) {
     d.world_efc[2 * w] = 0;
     d.world_efc[2 * w + 1] = 0;
@@ -155,13 +154,16 @@ __global__ void k_blocks_slots(mjhData d) {
     if (slot < d.world_efc[2 * w + 1]) d.efc_active[d.world_efc[2 * w] + slot] = r;
   }
 }
-// one wavefront per gathered world: the source rows in ascending order
+// one wavefront per world: a big world joins the big-world launch's map;
+// of a gathered world the source rows in ascending order
 // (rank sort from efc_active into efc_worldid of the new block), then the
 // rows' J, D and aref copied in that order; efc_worldid of the new block
 // keeps the source rows for the scatter
 __global__ void __launch_bounds__(64) k_blocks_gather(mjhData d, int nv) {
   const int w = blockIdx.x;
-  if (w >= d.nworld || !(d.world_flags[w] & kFlagGathered)) return;
+  if (w >= d.nworld) return;
+  if (threadIdx.x == 0) mark_big_world(d, w, d.world_efc[2 * w + 1]);
+  if (!(d.world_flags[w] & kFlagGathered)) return;
   const int b = d.world_efc[2 * w], n = d.world_efc[2 * w + 1];
   const int* src = d.efc_active + b;
   for (int i = threadIdx.x; i < n; i += 64) {
@@ -258,12 +260,19 @@ __global__ void __launch_bounds__(64) k_adjoint_state_grad(mjhModel m, mjhData d
   adjoint_state_grad(m, d, lam, g_qpos, g_qvel, g_act, t);
 }
 
+// dofs of a 32-lane model as its kernels pad them (with_nvc)
+int reg_nvc(int nv) { return nv > 0 && nv <= 28 ? (nv + 3) & ~3 : 32; }
+
 // per-block linear algebra (factor_m, solve_m, the integrators): the
 // largest kinematic tree's block and right-hand side staged in LDS, and
 // MuJoCo's sparse factor (nM) for sparse models
 int lds_linalg(const mjhModel& m) {
   const int b = m.tree_dof_max > 0 ? m.tree_dof_max : m.nv;
-  const int a = b * b + b;
+  int a = b * b + b;
+  if (m.nv <= kRegNvMax) {  // 32-lane teams stage whole matrices
+    const int r = lds_reg_matrix(reg_nvc(m.nv));
+    if (r > a) a = r;
+  }
   return m.opt.is_sparse && m.nM > a ? m.nM : a;
 }
 // the global-memory solver of the tail launches: per-block linear algebra
@@ -297,7 +306,15 @@ constexpr int kLdsRowsMin = 256, kLdsRowsMax = 1024;
 // defaults, MJH_SOLVER_WIDE=1 / 0 puts the Hessian of any 64-lane model in
 // efc_h / in LDS (where it fits).
 Tune tune_for(const mjhModel& m, bool reg) {
-  Tune t{64, reg ? 32 : 0, 0};
+  Tune t{64, 0, 0};
+  if (reg) {
+    // as many Jacobian rows as leave a CU twelve workgroups (three wavefronts
+    // per SIMD, what the registers allow), at least the nvc the solver's
+    // layout has anyway
+    const int nvc = reg_nvc(m.nv), room = (int)(lds_cap() / sizeof(float)) / 24;
+    t.rj = (room - lds_reg_floats(0, nvc, 2)) / reg_row_stride(nvc) + nvc;
+    if (t.rj < nvc) t.rj = nvc;
+  }
   if (!reg) {
     t.rmax = kLdsRowsMin;
     const int cap = (int)(lds_cap() / sizeof(float));
@@ -389,21 +406,22 @@ bool reg_path(const mjhModel& m) {
 // per-world LDS of the 32-lane kernels, a multiple of 4 floats so every
 // world's broadcast buffers are float4-aligned
 int lds_solve_reg(const mjhModel& m, const Tune& t) {
-  const int a = lds_reg_floats(t.rj, (m.nv + 3) & ~3), b = lds_linalg(m);
+  const int a = lds_reg_floats(t.rj, reg_nvc(m.nv), 2), b = lds_linalg(m);
   return ((a > b ? a : b) + 3) & ~3;
 }
 int lds_solve_reg(const mjhModel& m) { return lds_solve_reg(m, tune_for(m)); }
-// The register tail stages as many Jacobian rows as two worlds' LDS fit in
-// 64 KB (up to every row of kRegRows).
+// The big-world launch stages as many Jacobian rows as two worlds hold in a
+// quarter of a CU's LDS (40 KiB; 164 rows at nv 27), so that every SIMD gets
+// a wavefront.
 Tune tune_tail_reg(const mjhModel& m, Tune t) {
-  const int nvc = (m.nv + 3) & ~3;
-  const int fit = (16384 / 2 - lds_reg_floats(0, nvc) - 3) / (nvc + 1);
+  const int nvc = reg_nvc(m.nv);
+  const int fit = ((int)(lds_cap() / sizeof(float)) / 8 - lds_reg_floats(0, nvc, kRegSets)) / reg_row_stride(nvc) + nvc;
   t.rj = fit < kRegRows ? fit : kRegRows;
   return t;
 }
 Tune tune_tail_reg(const mjhModel& m) { return tune_tail_reg(m, tune_for(m)); }
 int lds_tail_reg(const mjhModel& m, const Tune& tail) {
-  const int a = lds_reg_floats(tail.rj, (m.nv + 3) & ~3), b = lds_linalg(m);
+  const int a = lds_reg_floats(tail.rj, reg_nvc(m.nv), kRegSets), b = lds_linalg(m);
   return ((a > b ? a : b) + 3) & ~3;
 }
 int lds_tail_reg(const mjhModel& m) { return lds_tail_reg(m, tune_tail_reg(m)); }
@@ -636,7 +654,6 @@ int do_step_fused(const mjhModel& m, const mjhData& d, hipStream_t s) {
 
 // one workgroup per group
 __global__ void k_reset_groups(const GroupDesc* __restrict__ g) {
-  if (threadIdx.x != 0) return;
   const GroupDesc& G = g[blockIdx.x];
   reset_counters(G.d, (G.m.opt.disableflags & mjhDSBL_CONSTRAINT) ? 1 : 3);
 }
@@ -736,15 +753,19 @@ int max_of(int a, int b) { return a > b ? a : b; }
 // model from device memory (the kernel-argument copy of the model compiles
 // to slower code for these kernels: part of it in scratch memory, more
 // registers, one wavefront per SIMD fewer).
-static_assert(sizeof(GroupDesc) <= MJH_STEP_DESC_WORDS * sizeof(int), "step_desc too small");
+static_assert(sizeof(GroupDesc) <= kBigMapWord * sizeof(int), "the description takes the first half of step_desc");
 static_assert(sizeof(GroupDesc) <= 4000, "the description must fit the kernel arguments");
 // writes the description and clears the step's counters (which as in
 // reset_counters) in one launch
 __global__ void k_write_desc(GroupDesc g, GroupDesc* out, int which) {
-  if (threadIdx.x == 0) {
-    *out = g;
-    reset_counters(g.d, which);
-  }
+  // lane-strided words of the argument, read where it lies (g itself indexed
+  // by lane would be copied to scratch memory first); one lane writing the
+  // whole struct took 6 us
+  typedef __attribute__((address_space(4))) const int kernarg;
+  kernarg* src = (kernarg*)__builtin_amdgcn_kernarg_segment_ptr();
+  int* dst = reinterpret_cast<int*>(out);
+  for (unsigned i = threadIdx.x; i < sizeof(GroupDesc) / sizeof(int); i += blockDim.x) dst[i] = src[i];
+  reset_counters(g.d, which);
 }
 // The description of d as the only group of a launch.
 GroupDesc single_desc(const mjhModel& m, const mjhData& d) {
@@ -764,7 +785,7 @@ int solve_reg_desc(const mjhModel& m, const mjhData& d, hipStream_t s) {
   if ((size_t)max_of(2 * l_solve, 2 * l_big) * sizeof(float) > lds_cap())
     return fail(MJH_ERR_CAPACITY, "solve: model too large for the dense LDS kernels (nv = " + std::to_string(m.nv) + ")");
   GroupDesc* dev = reinterpret_cast<GroupDesc*>(d.step_desc);
-  hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(64), 0, s, single_desc(m, d), dev, 0);
+  hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(256), 0, s, single_desc(m, d), dev, 0);
   TRY(check_launch("solve: description"));
   GroupTable t32;
   t32.dev = dev;
@@ -792,7 +813,7 @@ int do_step_fused_desc(const mjhModel& m, const mjhData& d, hipStream_t s) {
   if (need * sizeof(float) > lds_cap())
     return fail(MJH_ERR_CAPACITY,
                 "step_fused: model too large for the dense LDS kernels (nv = " + std::to_string(m.nv) + ")");
-  hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(64), 0, s, g, dev, (m.opt.disableflags & mjhDSBL_CONSTRAINT) ? 1 : 3);
+  hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(256), 0, s, g, dev, (m.opt.disableflags & mjhDSBL_CONSTRAINT) ? 1 : 3);
   TRY(check_launch("step_fused: description"));
   GroupTable t32, t64;
   t32.dev = t64.dev = dev;
@@ -1200,15 +1221,15 @@ int mjh_multi_step_static(int ngroups, const mjhModel* models, const mjhData* da
     const int nw = datas[i].nworld;
     if (c.reg) {
       gd.first_block = (int)b32;
-      hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(64), 0, s, gd, plan.t32.dev + i32, 0);
+      hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(256), 0, s, gd, plan.t32.dev + i32, 0);
       gd.first_block = (int)b32_64;
-      hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(64), 0, s, gd, plan.t32_64.dev + i32, 0);
+      hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(256), 0, s, gd, plan.t32_64.dev + i32, 0);
       b32 += (nw + 1) / 2;
       b32_64 += nw;
       i32++;
     } else {
       gd.first_block = (int)b64;
-      hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(64), 0, s, gd, plan.t64.dev + i64, 0);
+      hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(256), 0, s, gd, plan.t64.dev + i64, 0);
       b64 += nw;
       i64++;
     }

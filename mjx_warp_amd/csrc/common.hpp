@@ -246,6 +246,21 @@ MJH_DEV int dpp_i(int v) {
   return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
 }
 
+// The values of the even and of the odd 16-lane rows of v, each in both rows
+// of a pair (lane i gets lanes i & ~16 and i | 16): one v_permlane16_swap,
+// where a swizzle through the LDS hardware left the reduction waiting on it.
+struct SwapRows {
+  int even, odd;
+};
+MJH_DEV SwapRows swap_rows(int v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return SwapRows{(int)r[0], (int)r[1]};
+}
+MJH_DEV float add_rows(float v) {
+  const SwapRows r = swap_rows(__float_as_int(v));
+  return __int_as_float(r.even) + __int_as_float(r.odd);
+}
+
 // Sum over each 32-lane half of the wavefront (all lanes of a half get
 // identical bits: every step adds the same two rounded values in both lanes
 // of a pair).  The input is materialised first, so a product passed in is
@@ -258,17 +273,37 @@ MJH_DEV float sum32(float v) {
   v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]: lane ^ 2
   v += dpp_f<0x141>(v);  // row_half_mirror: 8-lane halves of a row
   v += dpp_f<0x140>(v);  // row_mirror: the two 8-lane halves of a row
-  // bitmask swizzle inside 32-lane groups: and 0x1f, or 0, xor 0x10
-  v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));
-  return v;
+  return add_rows(v);
+}
+// Two sums at once, each with the bits of sum32: the swap between the 16-lane
+// rows takes both, so that the pair costs two swaps where two sums take two
+// with the copies each needs of its operand.
+MJH_DEV void sum32_pair(float* x, float* y) {
+  float a = *x, b = *y;
+  asm volatile("" : "+v"(a));
+  asm volatile("" : "+v"(b));
+  a += dpp_f<0xB1>(a);
+  b += dpp_f<0xB1>(b);
+  a += dpp_f<0x4E>(a);
+  b += dpp_f<0x4E>(b);
+  a += dpp_f<0x141>(a);
+  b += dpp_f<0x141>(b);
+  a += dpp_f<0x140>(a);
+  b += dpp_f<0x140>(b);
+  // even rows: both rows of a; odd rows: both rows of b
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(a), __float_as_int(b), false, false);
+  const float s = __int_as_float((int)r[0]) + __int_as_float((int)r[1]);
+  const SwapRows t = swap_rows(__float_as_int(s));
+  *x = __int_as_float(t.even);
+  *y = __int_as_float(t.odd);
 }
 MJH_DEV int sum32_int(int v) {
   v += dpp_i<0xB1>(v);
   v += dpp_i<0x4E>(v);
   v += dpp_i<0x141>(v);
   v += dpp_i<0x140>(v);
-  v += __builtin_amdgcn_ds_swizzle(v, 0x401F);
-  return v;
+  const SwapRows r = swap_rows(v);
+  return r.even + r.odd;
 }
 
 // Sum of v over the TEAM lanes of a team; every lane gets the same bits

@@ -57,6 +57,62 @@ __host__ __device__ constexpr int lds_constraint_floats() {
   return 29 * TEAM;
 }
 
+// Worlds that the 32-lane solve launches leave to the big-world launch: more
+// rows than their two row sets hold, at most kBigRowsMax.
+constexpr int kBigRowsMin = 2 * kRegTeam, kBigRowsMax = 256;
+MJH_DEV bool big_rows(int nr) { return nr > kBigRowsMin && nr <= kBigRowsMax; }
+
+// The big-world launch's map: a bit per world, set when its rows are built,
+// in the second half of Data.step_desc (the description takes the first);
+// null without one or with more worlds than it has bits, and the launch then
+// looks for its worlds in place.  By the map two such worlds share every
+// wavefront of that launch; in place, with one world in twelve big, nearly
+// all its wavefronts held one (24,576 humanoids: 2.65 ms against 1.41 ms).
+constexpr int kBigMapWord = MJH_STEP_DESC_WORDS / 2;
+constexpr int kBigMapWorlds = 32 * (MJH_STEP_DESC_WORDS - kBigMapWord);
+MJH_DEV unsigned* big_map(const mjhData& d) {
+  return d.step_desc && d.nworld <= kBigMapWorlds ? reinterpret_cast<unsigned*>(d.step_desc) + kBigMapWord : nullptr;
+}
+MJH_DEV void mark_big_world(const mjhData& d, int w, int nr) {
+  unsigned* map = big_map(d);
+  if (map && big_rows(nr)) atomicOr(map + w / 32, 1u << (w % 32));
+}
+// cleared by n threads, of which this is the i-th
+MJH_DEV void clear_big_map(const mjhData& d, int i, int n) {
+  if (unsigned* map = big_map(d))
+    for (int k = i; k < (d.nworld + 31) / 32; k += n) map[k] = 0;
+}
+// The i-th world of the map, or -1 past the last; every lane of the
+// wavefront calls it, i may differ per lane.  Lane l counts the l-th run of
+// words; the run that holds world i is then walked.
+MJH_DEV int big_map_world(const mjhData& d, const unsigned* map, int i) {
+  const int words = (d.nworld + 31) / 32, run = (words + 63) / 64, lane = threadIdx.x & 63;
+  int mine = 0;
+  for (int k = lane * run; k < (lane + 1) * run && k < words; k++) mine += __popc(map[k]);
+  int total;
+  const int before = team_exscan_int<64>(mine, lane, &total);
+  if (__ballot(i < total) == 0) return -1;
+  int owner = 0, skip = 0;  // the last run that starts at or before world i
+  for (int l = 0; l < 64; l++) {
+    const int b = __shfl(before, l), m = __shfl(mine, l);
+    if (m > 0 && b <= i) {
+      owner = l;
+      skip = b;
+    }
+  }
+  if (i >= total) return -1;
+  for (int k = owner * run;; k++) {
+    unsigned bits = map[k];
+    const int n = __popc(bits);
+    if (skip + n <= i) {
+      skip += n;
+      continue;
+    }
+    for (; skip < i; skip++) bits &= bits - 1;
+    return 32 * k + __ffs(bits) - 1;
+  }
+}
+
 // The rows of one world into the block [base, base + total) of the pool
 // (reserved by the caller; total counts nlim limit rows first): limit rows
 // in joint order, then four rows per active contact in contact order, as
@@ -82,6 +138,7 @@ MJH_DEV void make_constraint_rows(const mjhModel& m, const mjhData& d, float* ld
     d.world_efc[2 * w] = base;
     d.world_efc[2 * w + 1] = nwritten;
     if (base + total > cap) atomicAdd(d.overflow + 2, min(total, base + total - cap));
+    if (TEAM == kRegTeam) mark_big_world(d, w, nwritten);
   }
   // limit rows (constraint.py:104-141)
   int k0 = 0;

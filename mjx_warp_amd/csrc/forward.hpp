@@ -199,11 +199,11 @@ MJH_DEV void mul_m(const mjhModel& m, const float* qM, float* res, const float* 
   });
 }
 
-// forward.py:43-162 _advance (without the host-side time update)
+// forward.py:43-162 _advance (without the host-side time update), in parts:
+// the activations ...
 template <int TEAM>
-MJH_DEV void advance(const mjhModel& m, const mjhData& d, const float* qacc_all, const Team<TEAM>& t) {
-  if (!t.valid) return;
-  const int w = t.world, nv = m.nv;
+MJH_DEV void advance_act(const mjhModel& m, const mjhData& d, const Team<TEAM>& t) {
+  const int w = t.world;
   const float dt = m.opt.timestep;
   if (m.na) {
     float* act = WPTR(d.act, w, m.na);
@@ -224,11 +224,12 @@ MJH_DEV void advance(const mjhModel& m, const mjhData& d, const float* qacc_all,
       act[adr] = x;
     }
   }
-  float* qvel = WPTR(d.qvel, w, nv);
-  const float* qacc = WPTR(qacc_all, w, nv);
-  for (int i = t.lane; i < nv; i += TEAM) qvel[i] = qvel[i] + qacc[i] * dt;
-  sync();
-  float* qpos = WPTR(d.qpos, w, m.nq);
+}
+// ... the positions, by the world's new velocities qvel (global or LDS) ...
+template <int TEAM>
+MJH_DEV void advance_qpos(const mjhModel& m, const mjhData& d, const float* qvel, const Team<TEAM>& t) {
+  const float dt = m.opt.timestep;
+  float* qpos = WPTR(d.qpos, t.world, m.nq);
   for (int j = t.lane; j < m.njnt; j += TEAM) {
     const int jt = m.jnt_type[j], qa = m.jnt_qposadr[j], da = m.jnt_dofadr[j];
     if (jt == mjhJNT_FREE) {
@@ -242,6 +243,20 @@ MJH_DEV void advance(const mjhModel& m, const mjhData& d, const float* qacc_all,
       qpos[qa] = qpos[qa] + dt * qvel[da];
     }
   }
+}
+
+// ... and all of it from the accelerations qacc_all
+template <int TEAM>
+MJH_DEV void advance(const mjhModel& m, const mjhData& d, const float* qacc_all, const Team<TEAM>& t) {
+  if (!t.valid) return;
+  const int w = t.world, nv = m.nv;
+  const float dt = m.opt.timestep;
+  advance_act(m, d, t);
+  float* qvel = WPTR(d.qvel, w, nv);
+  const float* qacc = WPTR(qacc_all, w, nv);
+  for (int i = t.lane; i < nv; i += TEAM) qvel[i] = qvel[i] + qacc[i] * dt;
+  sync();
+  advance_qpos(m, d, qvel, t);
 }
 
 // forward.py:165-242 euler (dense eulerdamp: (M + dt diag(damping)) qacc =
@@ -277,6 +292,105 @@ MJH_DEV bool advances_with_qacc(const mjhModel& m) {
   return !passive_on && !act_on;
 }
 
+// forward.py:278-299: the actuators' velocity derivatives
+template <int TEAM>
+MJH_DEV void actuator_vel_derivative(const mjhModel& m, const mjhData& d, const Team<TEAM>& t) {
+  const int w = t.world, nu = m.nu;
+  float* avi = WPTR(d.act_vel_integration, w, nu);
+  const float* ctrl = WPTR(d.ctrl, w, nu);
+  const float* act = WPTR(d.act, w, m.na);
+  for (int a = t.lane; a < nu; a += TEAM) {
+    float bv = 0.0f, gv = 0.0f;
+    if (m.actuator_biastype[a] == mjhBIAS_AFFINE) bv = m.actuator_biasprm[10 * a + 2];
+    if (m.actuator_gaintype[a] == mjhGAIN_AFFINE) gv = m.actuator_gainprm[10 * a + 2];
+    // the reference indexes act by actuator id here (forward.py:296-297)
+    const float c = (m.actuator_dyntype[a] != mjhDYN_NONE) ? act[a] : ctrl[a];
+    avi[a] = bv + gv * c;
+  }
+}
+
+// Euler or implicitfast of one world on a 32-lane team, given the lane's
+// acceleration and its forces qs + qc: the integration matrix's row
+// (M + dt diag(damping), or with actuator derivatives qM - dt (moment'
+// diag(vel) moment - diag(damping))) and its factor in registers.  rows: M
+// as stage_sym leaves it, whose diagonal takes the damping there and whose
+// room the matrix is stored from; blocks: select the lane's block of M (a
+// caller's M; crb's has zeros elsewhere); cbuf: a broadcast buffer, through
+// which the velocities pass to the positions.
+template <int NVC>
+MJH_DEV void integrate_reg(const mjhModel& m, const mjhData& d, bool euler_step, float qacc, float force, float* cbuf,
+                           float* rows, int beg, int end, bool blocks, const Team<kRegTeam>& t) {
+  const int w = t.world, nv = m.nv, nu = m.nu, lane = t.lane;
+  const bool dof = lane < nv;
+  float acc = qacc;
+  if (!advances_with_qacc(m)) {
+    const bool damping = euler_step || !(m.opt.disableflags & mjhDSBL_PASSIVE);
+    const bool act_on = !euler_step && !(m.opt.disableflags & mjhDSBL_ACTUATION) && m.actuator_affine_bias_gain;
+    const float* avi = WPTR(d.act_vel_integration, w, nu);
+    if (act_on) {
+      actuator_vel_derivative(m, d, t);
+      sync();
+    }
+    const float damp = (dof && damping) ? m.dof_damping[lane] * m.opt.timestep : 0.0f;
+    RegChol<NVC> c{lane, cbuf};
+    if (dof) rows[lane * c.JS + lane] += damp;
+    if (blocks && lane < NVC)
+      for (int j = 0; j < NVC; j++)
+        if (j != lane && (j < beg || j >= end)) rows[lane * c.JS + j] = 0.0f;
+    wave_fence();
+    c.load_rows(rows);
+    if (act_on) {
+      const float* moment = WPTR(d.actuator_moment, w, nu * nv);
+      for (int a = 0; a < nu; a++) {
+        const float* mr = moment + a * nv;
+        const float ca = dof ? m.opt.timestep * mr[lane] * avi[a] : 0.0f;
+        if (ca == 0.0f) continue;
+#pragma unroll
+        for (int j = 0; j < NVC; j++)
+          if (j < nv && j >= beg && j < end) c.h[j] -= ca * mr[j];
+      }
+    }
+    if (!euler_step) {
+      if (dof) d.qfrc_integration[w * nv + lane] = force;
+      float* const qMi = WPTR(d.qM_integration, w, nv * nv);
+      if (act_on) c.store_rows(qMi, nv, beg, end, rows, false);
+      else store_blocks<NVC>(qMi, nv, beg, end, lane, rows, false);
+    }
+    c.template factor<false>(!euler_step);
+    acc = c.solve(force);
+    if (dof) d.qacc_integration[w * nv + lane] = acc;
+  }
+  advance_act(m, d, t);
+  const float v = dof ? d.qvel[w * nv + lane] + acc * m.opt.timestep : 0.0f;
+  if (dof) d.qvel[w * nv + lane] = v;
+  wave_fence();
+  cbuf[lane] = v;
+  wave_fence();
+  advance_qpos(m, d, cbuf, t);
+}
+
+// the integrator launches' form of it: M from global memory; lds:
+// lds_reg_matrix
+MJH_DEV void integrate_reg(const mjhModel& m, const mjhData& d, bool euler_step, float* lds, const Team<kRegTeam>& t) {
+  if (t.valid) {
+    const int w = t.world, nv = m.nv, lane = t.lane;
+    const bool dof = lane < nv;
+    int beg, end;
+    tree_block(m, lane, &beg, &end);
+    const bool with_qacc = advances_with_qacc(m);
+    const float qacc = dof && with_qacc ? d.qacc[w * nv + lane] : 0.0f;
+    const float force = dof && !with_qacc ? d.qfrc_smooth[w * nv + lane] + d.qfrc_constraint[w * nv + lane] : 0.0f;
+    with_nvc(nv, [&](auto nvc) {
+      constexpr int NVC = decltype(nvc)::value;
+      float* const rows = lds + kRegLdsMin;
+      if (!with_qacc) stage_sym<NVC>(WPTR(d.qMd, w, nv * nv), nv, lane, rows);
+      integrate_reg<NVC>(m, d, euler_step, qacc, force, lds, rows, beg, end, true, t);
+      return 0;
+    });
+  }
+  sync();
+}
+
 template <int TEAM>
 MJH_DEV void euler(const mjhModel& m, const mjhData& d, float* lds, const Team<TEAM>& t) {
   const int w = t.world, nv = m.nv;
@@ -287,26 +401,7 @@ MJH_DEV void euler(const mjhModel& m, const mjhData& d, float* lds, const Team<T
   }
   if (m.opt.is_sparse) euler_sparse_outputs(m, d, lds, t);
   if constexpr (TEAM == kRegTeam) {
-    // (M + dt diag(damping)) qacc_int = qfrc_smooth + qfrc_constraint, the
-    // matrix row and its factor in registers
-    if (t.valid) {
-      const int lane = t.lane;
-      const bool dof = lane < nv;
-      int beg, end;
-      tree_block(m, lane, &beg, &end);
-      const float damp = dof ? m.dof_damping[lane] * m.opt.timestep : 0.0f;
-      const float b = dof ? d.qfrc_smooth[w * nv + lane] + d.qfrc_constraint[w * nv + lane] : 0.0f;
-      const float x = with_nvc(nv, [&](auto nvc) {
-        RegChol<decltype(nvc)::value> c{lane, lds};
-        c.load_sym(WPTR(d.qMd, w, nv * nv), nv, beg, end, damp);
-        c.factor();
-        return c.solve(b);
-      });
-      if (dof) d.qacc_integration[w * nv + lane] = x;
-    }
-    sync();
-    advance(m, d, d.qacc_integration, t);
-    sync();
+    integrate_reg(m, d, true, lds, t);
     return;
   }
   if (t.valid) {
@@ -349,62 +444,13 @@ MJH_DEV void implicit(const mjhModel& m, const mjhData& d, float* lds, const Tea
     return;
   }
   const float dt = m.opt.timestep;
-  float* avi = WPTR(d.act_vel_integration, w, nu);
-  if (act_on && t.valid) {
-    const float* ctrl = WPTR(d.ctrl, w, nu);
-    const float* act = WPTR(d.act, w, m.na);
-    for (int a = t.lane; a < nu; a += TEAM) {
-      float bv = 0.0f, gv = 0.0f;
-      if (m.actuator_biastype[a] == mjhBIAS_AFFINE) bv = m.actuator_biasprm[10 * a + 2];
-      if (m.actuator_gaintype[a] == mjhGAIN_AFFINE) gv = m.actuator_gainprm[10 * a + 2];
-      // the reference indexes act by actuator id here (forward.py:296-297)
-      const float c = (m.actuator_dyntype[a] != mjhDYN_NONE) ? act[a] : ctrl[a];
-      avi[a] = bv + gv * c;
-    }
-  }
-  sync();
   if constexpr (TEAM == kRegTeam) {
-    // qM_integration = qM - dt (moment' diag(vel) moment - diag(damping)),
-    // a row per lane in registers, written out, factored and solved in place
-    if (t.valid) {
-      const int lane = t.lane;
-      const bool dof = lane < nv;
-      int beg, end;
-      tree_block(m, lane, &beg, &end);
-      const float damp = (dof && passive_on) ? m.dof_damping[lane] * dt : 0.0f;
-      const float b = dof ? d.qfrc_smooth[w * nv + lane] + d.qfrc_constraint[w * nv + lane] : 0.0f;
-      if (dof) d.qfrc_integration[w * nv + lane] = b;
-      const float* moment = WPTR(d.actuator_moment, w, nu * nv);
-      float* qMi = WPTR(d.qM_integration, w, nv * nv);
-      const float x = with_nvc(nv, [&](auto nvc) {
-        constexpr int NVC = decltype(nvc)::value;
-        RegChol<NVC> c{lane, lds};
-        c.load_sym(WPTR(d.qMd, w, nv * nv), nv, beg, end, damp);
-        if (act_on) {
-          for (int a = 0; a < nu; a++) {
-            const float* mr = moment + a * nv;
-            const float ca = dof ? dt * mr[lane] * avi[a] : 0.0f;
-            if (ca == 0.0f) continue;
-#pragma unroll
-            for (int j = 0; j < NVC; j++)
-              if (j < nv && j >= beg && j < end) c.h[j] -= ca * mr[j];
-          }
-        }
-        if (dof) {
-#pragma unroll
-          for (int j = 0; j < NVC; j++)
-            if (j >= beg && j < end) qMi[lane * nv + j] = c.h[j];
-        }
-        c.factor();
-        return c.solve(b);
-      });
-      if (dof) d.qacc_integration[w * nv + lane] = x;
-    }
-    sync();
-    advance(m, d, d.qacc_integration, t);
-    sync();
+    integrate_reg(m, d, false, lds, t);
     return;
   }
+  const float* avi = WPTR(d.act_vel_integration, w, nu);
+  if (act_on && t.valid) actuator_vel_derivative(m, d, t);
+  sync();
   if (t.valid) {
     const float* qM = WPTR(d.qMd, w, nv * nv);
     const float* moment = WPTR(d.actuator_moment, w, nu * nv);

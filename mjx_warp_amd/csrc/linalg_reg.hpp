@@ -25,6 +25,14 @@ constexpr int kRegNvMax = 32;
 // buffer (one float per lane)
 constexpr int kRegLdsMin = 32;
 
+// Row stride of nvc-column rows staged in LDS (matrix rows, Jacobian rows):
+// an odd number of float4s (nvc or nvc + 4), so that a row is read as float4s
+// -- by every lane at once (the Hessian's rank-1 updates) or a row per lane
+// without bank conflicts -- and a column entry per lane stays conflict free.
+__host__ __device__ constexpr int reg_row_stride(int nvc) { return (nvc / 4) % 2 ? nvc : nvc + 4; }
+// LDS floats of the broadcast buffer and one staged matrix
+__host__ __device__ constexpr int lds_reg_matrix(int nvc) { return kRegLdsMin + nvc * reg_row_stride(nvc); }
+
 MJH_DEV void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -50,6 +58,14 @@ MJH_DEV gfloat* opaque(const float* p) {
 MJH_DEV int opaque(int i) {
   asm volatile("" : "+v"(i));
   return i;
+}
+
+// v, computed before any memory access that follows: keeps the compiler from
+// issuing the loads of several dot products together, whose operands then
+// hold the registers of another wavefront per SIMD (200 VGPRs against 150).
+MJH_DEV float settle(float v) {
+  asm volatile("" : "+v"(v) : : "memory");
+  return v;
 }
 
 // Calls f(std::integral_constant<int, NVC>) with NVC = nv rounded up to 4.
@@ -79,6 +95,19 @@ MJH_DEV void tree_block(const mjhModel& m, int dof, int* beg, int* end) {
   });
 }
 
+// Staged rows (stride reg_row_stride(NVC)) into the blocks [beg, end) of A
+// (global, [nv, nv]), a row at a time with lanes over columns (a column's
+// block holds the rows [beg, end) too); lower: zeros above the diagonal.
+template <int NVC>
+MJH_DEV void store_blocks(float* A, int nv, int beg, int end, int lane, const float* rows, bool lower) {
+  if (lane < nv) {
+#pragma unroll 4
+    for (int r = 0; r < nv; r++)
+      if (r >= beg && r < end) A[r * nv + lane] = (lower && lane > r) ? 0.0f : rows[r * reg_row_stride(NVC) + lane];
+  }
+  wave_fence();
+}
+
 template <int NVC>
 struct RegChol {
   static_assert(NVC % 4 == 0 && NVC <= kRegNvMax, "padded dof count");
@@ -102,75 +131,169 @@ struct RegChol {
     rdiag = 1.0f;
   }
 
-  // A lower factor row read from global memory (L[lane * nv + j], j within
-  // the lane's block, up to the diagonal).
-  MJH_DEV void load_lower(const float* L, int nv, int beg) {
+  static constexpr int JS = reg_row_stride(NVC);
+  // the staged row this lane reads: its own (lanes past the padding read the
+  // last row; nothing they derive from it reaches another lane)
+  MJH_DEV const float4* row4(const float* rows) const {
+    return reinterpret_cast<const float4*>(rows + (lane < NVC ? lane : NVC - 1) * JS);
+  }
+
+  // Row `lane` of a matrix staged by stage_sym, of a mass matrix that crb
+  // wrote: entries of dofs in different trees are zero, so no block to select.
+  MJH_DEV void load_rows(const float* rows) {
+    const float4* r = row4(rows);
+#pragma unroll
+    for (int q = 0; q < NVC / 4; q++) {
+      const float4 v = r[q];
+      h[4 * q] = v.x;
+      h[4 * q + 1] = v.y;
+      h[4 * q + 2] = v.z;
+      h[4 * q + 3] = v.w;
+    }
+    rdiag = 1.0f;
+  }
+
+  // The lower factor's row `lane` from global memory, restricted to the
+  // lane's block (from column beg up to the diagonal), by way of the staging
+  // buffer `rows` (NVC rows): a row per lane read in place touches a cache
+  // line per lane with every load.
+  MJH_DEV void load_lower(const float* L, int nv, int beg, float* rows) {
+    gfloat* Lc = opaque(L) + (lane < nv ? lane : 0);
+    wave_fence();
+    if (lane < NVC) {
+#pragma unroll 7
+      for (int r = 0; r < nv; r++) rows[r * JS + lane] = Lc[r * nv];
+    }
+    wave_fence();
+    const float4* r4 = row4(rows);
     const int ln = opaque(lane);
     const bool dof = ln < nv;
-    gfloat* Lr = opaque(L) + (dof ? ln * nv : 0);
 #pragma unroll
-    for (int j = 0; j < NVC; j++) {
-      const float v = Lr[j < nv ? j : 0];
-      h[j] = (dof && j >= beg && j <= ln) ? v : (j == ln ? 1.0f : 0.0f);
+    for (int q = 0; q < NVC / 4; q++) {
+      const float4 v = r4[q];
+      const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int j = 4 * q + u;
+        h[j] = (dof && j >= beg && j <= ln) ? e[u] : (j == ln ? 1.0f : 0.0f);
+      }
     }
-    rdiag = dof ? 1.0f / Lr[ln] : 1.0f;
+    rdiag = dof ? 1.0f / rows[ln * JS + ln] : 1.0f;
+    wave_fence();
   }
+  // rdiag as load_lower sets it, from a factor that store_rows staged
+  MJH_DEV void divide_diag(const float* rows, int nv) { rdiag = lane < nv ? 1.0f / rows[lane * JS + lane] : 1.0f; }
 
   // Cholesky H = L L' of the lane-owned rows (right-looking, one column
   // broadcast through LDS per step).  Lane i keeps L[i][0..i] in h[0..i]
   // and 1 / L[i][i] in rdiag.
-  MJH_DEV void factor() {
+  // kDiag unset: the diagonal of L is not kept, for a factor that solve()
+  // alone reads.  rsq: 1 / L[i][i] from one reciprocal square root, which
+  // differs from square root and reciprocal in the last bit (callers keep the
+  // form they have, so that their results stay as they are).
+  template <bool kDiag = true>
+  MJH_DEV void factor(bool rsq = false) {
+    // this call's own lane number: comparisons with it are made where they
+    // are used instead of being kept in (and spilled from) scalar registers
+    const int ln = opaque(lane);
 #pragma unroll
     for (int k = 0; k < NVC; k++) {
       wave_fence();
-      cbuf[lane] = h[k];
+      cbuf[ln] = h[k];
       wave_fence();
-      const float dkk = cbuf[k];
-      const float lkk = __builtin_amdgcn_sqrtf(dkk);
-      const float inv = __builtin_amdgcn_rcpf(lkk);
-      // L[i][k] L[j][k] = H[i][k] H[j][k] / dkk
-      const float g = lane > k ? h[k] * (inv * inv) : 0.0f;
+      float c[NVC];
 #pragma unroll
-      for (int j = k + 1; j < NVC; j++) h[j] = fmaf(-g, cbuf[j], h[j]);
-      if (lane == k) rdiag = inv;
-      h[k] = lane > k ? h[k] * inv : (lane == k ? lkk : h[k]);
+      for (int q = k / 4; q < NVC / 4; q++) {
+        const float4 v = reinterpret_cast<const float4*>(cbuf)[q];
+        c[4 * q] = v.x;
+        c[4 * q + 1] = v.y;
+        c[4 * q + 2] = v.z;
+        c[4 * q + 3] = v.w;
+      }
+      const float dkk = c[k];
+      float lkk = __builtin_amdgcn_sqrtf(dkk);
+      asm volatile("" : "+v"(lkk));  // else the compiler may make a rsq of the two
+      const float inv = rsq ? __builtin_amdgcn_rsqf(dkk) : __builtin_amdgcn_rcpf(lkk);
+      // L[i][k] L[j][k] = H[i][k] H[j][k] / dkk
+      const float g = ln > k ? h[k] * (inv * inv) : 0.0f;
+#pragma unroll
+      for (int j = k + 1; j < NVC; j++) h[j] = fmaf(-g, c[j], h[j]);
+      if (ln == k) rdiag = inv;
+      if (kDiag) h[k] = ln > k ? h[k] * inv : (ln == k ? lkk : h[k]);
+      else h[k] *= inv;  // solve() reads it in the lanes past k only
     }
   }
 
   // x = inv(L L') b with L from factor() / load_lower(); b, x one entry per
   // lane (padding lanes carry 0)
   MJH_DEV float solve(float b) const {
+    const int ln = opaque(lane);
     // forward: y = inv(L) b, column by column
     float y = b;
 #pragma unroll
     for (int k = 0; k < NVC; k++) {
       const float yk = bcast32(y * rdiag, k);
-      y = lane > k ? fmaf(-h[k], yk, y) : y;
+      y = ln > k ? fmaf(-h[k], yk, y) : y;
     }
     y *= rdiag;
     // backward: x = inv(L') y, x[k] = (y[k] - sum_{j>k} L[j][k] x[j]) / L[k][k]
     float x = 0.0f;
 #pragma unroll
     for (int k = NVC - 1; k >= 0; k--) {
-      const float s = sum32(lane > k ? h[k] * x : 0.0f);
-      if (lane == k) x = (y - s) * rdiag;
+      const float s = sum32(ln > k ? h[k] * x : 0.0f);
+      if (ln == k) x = (y - s) * rdiag;
     }
     return x;
   }
 
-  // Writes the factor's rows into L (global, [nv, nv]): the lower triangle of
-  // the lane's block [beg, end) and zeros above the diagonal inside the
-  // block, as the reference's tile factor (smooth.py:353-379).
-  MJH_DEV void store_block(float* L, int nv, int beg, int end) const {
-    if (lane >= nv) return;
-    float* Lr = L + lane * nv;
+  // Writes the rows into the blocks [beg, end) of A (global, [nv, nv]) by
+  // way of the staging buffer `rows` (NVC rows): stored a row at a time with
+  // lanes over columns, where a row per lane sent every word to the cache as
+  // a request of its own.  lower: the factor's lower triangle and zeros above
+  // the diagonal inside a block, as the reference's tile factor
+  // (smooth.py:353-379).
+  MJH_DEV void store_rows(float* A, int nv, int beg, int end, float* rows, bool lower) const {
+    wave_fence();
+    if (lane < NVC) {
+      float4* r4 = reinterpret_cast<float4*>(rows + lane * JS);
 #pragma unroll
-    for (int j = 0; j < NVC; j++)
-      if (j >= beg && j < end) Lr[j] = j <= lane ? h[j] : 0.0f;
+      for (int q = 0; q < NVC / 4; q++) r4[q] = make_float4(h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
+    }
+    wave_fence();
+    store_blocks<NVC>(A, nv, beg, end, lane, rows, lower);
   }
 };
 
-// qLD = tree-block Cholesky factors of qM, in registers (32-lane teams)
+// Stages the symmetric matrix A (global, [nv, nv]) into LDS rows (NVC rows
+// of stride reg_row_stride(NVC)), padded with identity rows: lane i loads
+// column i, coalesced across the team, as row i.
+template <int NVC>
+MJH_DEV void stage_sym(const float* A, int nv, int lane, float* rows) {
+  const int ln = opaque(lane);
+  gfloat* Ac = opaque(A) + (ln < nv ? ln : 0);
+  float4 v[NVC / 4];
+#pragma unroll
+  for (int q = 0; q < NVC / 4; q++) {
+    float e[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int j = 4 * q + u;
+      const float a = Ac[(j < nv ? j : 0) * nv];
+      e[u] = (ln < nv && j < nv) ? a : (j == ln ? 1.0f : 0.0f);
+    }
+    v[q] = make_float4(e[0], e[1], e[2], e[3]);
+  }
+  wave_fence();
+  if (ln < NVC) {
+    float4* r4 = reinterpret_cast<float4*>(rows + ln * reg_row_stride(NVC));
+#pragma unroll
+    for (int q = 0; q < NVC / 4; q++) r4[q] = v[q];
+  }
+  wave_fence();
+}
+
+// qLD = tree-block Cholesky factors of qM, in registers (32-lane teams);
+// lds: lds_reg_matrix
 MJH_DEV void reg_factor_blocks(const mjhModel& m, const float* M, float* L, float* lds, const Team<kRegTeam>& t) {
   const int nv = m.nv;
   int beg, end;
@@ -179,21 +302,22 @@ MJH_DEV void reg_factor_blocks(const mjhModel& m, const float* M, float* L, floa
     RegChol<decltype(nvc)::value> c{t.lane, lds};
     c.load_sym(M, nv, beg, end);
     c.factor();
-    c.store_block(L, nv, beg, end);
+    c.store_rows(L, nv, beg, end, lds + kRegLdsMin, true);
     return 0;
   });
 }
 
 // x = inv(M) y from the tree-block factor L (qLD), in registers; x may
-// alias y
-MJH_DEV void reg_solve_blocks(const mjhModel& m, const float* L, float* x, const float* y, const Team<kRegTeam>& t) {
+// alias y; lds: lds_reg_matrix
+MJH_DEV void reg_solve_blocks(const mjhModel& m, const float* L, float* x, const float* y, float* lds,
+                              const Team<kRegTeam>& t) {
   const int nv = m.nv;
   int beg, end;
   tree_block(m, t.lane, &beg, &end);
   const float b = t.lane < nv ? y[t.lane] : 0.0f;
   const float r = with_nvc(nv, [&](auto nvc) {
-    RegChol<decltype(nvc)::value> c{t.lane, nullptr};
-    c.load_lower(L, nv, beg);
+    RegChol<decltype(nvc)::value> c{t.lane, lds};
+    c.load_lower(L, nv, beg, lds + kRegLdsMin);
     return c.solve(b);
   });
   if (t.lane < nv) x[t.lane] = r;

@@ -557,7 +557,7 @@ template <int TEAM>
 MJH_DEV void solve_blocks(const mjhModel& m, const float* L, float* x, const float* y, float* lds,
                           const Team<TEAM>& t) {
   if constexpr (TEAM == kRegTeam) {
-    reg_solve_blocks(m, L, x, y, t);
+    reg_solve_blocks(m, L, x, y, lds, t);
     return;
   }
   const int nv = m.nv;

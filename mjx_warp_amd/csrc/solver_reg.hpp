@@ -3,15 +3,17 @@
 // _linesearch_iterative / _linesearch_parallel, CG beta, _done).
 //
 // Mapping: a team of 32 lanes per world, two worlds per wavefront.  Lane i
-// owns dof i -- its entries of qacc, Ma, grad, Mgrad, search, mv, the mass
-// matrix row (M is symmetric, so the row is read as a coalesced column) and
-// row i of the Newton Hessian and of its Cholesky factor, all in VGPRs.  Lane
+// owns dof i -- its entries of qacc, Ma, grad, Mgrad, search, mv and row i of
+// the Newton Hessian and of its Cholesky factor, all in VGPRs; its row of the
+// mass matrix is staged in LDS once and read there by every product with M,
+// every Hessian and the integrator.  Lane
 // r also owns constraint rows r, r + 32, ..., r + 32 (RS - 1) (Jaref, jv, D,
 // force and the line-search quadratic): RS row sets, of which the first
 // ceil(nr / 32) are live.  The world's Jacobian rows are staged in LDS with
-// the odd row stride NVC + 1, so both row-wise (lane = row) and column-wise
-// (lane = dof) reads are bank-conflict free; rows past the staged count are
-// read from global memory, where they are read-only during the solve.
+// a stride of an odd number of float4s (reg_row_stride): rows are read as
+// float4s and both row-wise (lane = row) and column-wise (lane = dof) reads
+// are bank-conflict free; rows past the staged count are read from global
+// memory, where they are read-only during the solve.
 //
 // Cross-lane sums are DPP butterflies inside 16-lane rows plus one swizzle
 // across the two rows of a team; every lane of the team ends with the same
@@ -26,6 +28,7 @@
 // count and no guards; padded entries never change a sum.
 #pragma once
 
+#include "constraint.hpp"
 #include "linalg_reg.hpp"
 #include "solver_lds.hpp"
 
@@ -33,11 +36,15 @@ namespace mjh {
 
 constexpr int kRegSets = 8;                // most row sets per lane
 constexpr int kRegRows = 32 * kRegSets;    // row capacity of the register solver
+static_assert(kRegRows == kBigRowsMax, "the big-world launch takes what the list holds");
 
-// LDS floats per world: broadcast buffers (vector 32, column 32, rows
-// kRegRows) and rj staged Jacobian rows of stride nvc + 1 (nvc: nv rounded
-// up to 4), rounded up to a float4.
-__host__ __device__ inline int lds_reg_floats(int rj, int nvc) { return (64 + kRegRows + rj * (nvc + 1) + 3) & ~3; }
+// LDS floats per world of the register solver with rs row sets: broadcast
+// buffers (vector 32, column 32, rows 32 rs), the mass matrix (nvc rows; nvc:
+// nv rounded up to 4) and rj staged Jacobian rows, whose room also stages
+// matrix rows on their way to global memory (at least nvc rows).
+__host__ __device__ constexpr int lds_reg_floats(int rj, int nvc, int rs) {
+  return 64 + 32 * rs + (nvc + (rj > nvc ? rj : nvc)) * reg_row_stride(nvc);
+}
 
 template <int NVC, int RS>
 struct RegSolver {
@@ -48,16 +55,15 @@ struct RegSolver {
   int w, nv, radr, nr, lane, rj;
   float* vbuf;  // [32] dof-vector broadcast
   float* fbuf;  // [32 * RS] row-scalar broadcast
-  float* Jl;    // [rj][JS] staged Jacobian rows
-  static constexpr int JS = NVC + 1;
-  const float* M;  // qM of the world (global, read-only during the solve)
+  const float* Ml;  // [NVC][JS] the mass matrix's rows
+  float* Jl;        // [rj][JS] staged Jacobian rows
+  static constexpr int JS = reg_row_stride(NVC);
   // dof lane state
   RegChol<NVC> ch;  // Hessian row and its Cholesky factor (CG: factor of M)
   float qacc, Ma, grad, Mgrad, search, mv, qs, qas, qc;
   // row lane state: rows lane + 32 s, s < RS
   float Jaref[RS], jv[RS], D[RS], force[RS], q0[RS], q1[RS], q2[RS];
 
-  int blk;   // CG: first dof of the lane's tree block
   int nset;  // live row sets, ceil(nr / 32) but at least 1 (team-uniform); set 0
              // is always live, which the loops state at compile time
   // the factor in ch is current: Newton's H = M + J' D(active) J depends on
@@ -78,14 +84,23 @@ struct RegSolver {
   }
   MJH_DEV float4 vec4(int q) const { return reinterpret_cast<const float4*>(vbuf)[q]; }
 
-  // M[lane] . v for the vector last passed to put_vec (M symmetric: the
-  // lane reads column `lane`, coalesced across the team)
+  // columns 4 q .. 4 q + 3 of staged row r
+  MJH_DEV float4 jrow4(int r, int q) const { return reinterpret_cast<const float4*>(Jl + r * JS)[q]; }
+
+  // M[lane] . v for the vector last passed to put_vec
   MJH_DEV float mrow_dot() const {
     float s = 0.0f;
-    if (lane >= nv) return s;
-    gfloat* Mc = opaque(M) + lane;
-    for (int j = 0; j < nv; j++) s += Mc[j * nv] * vbuf[j];
-    return s;
+    const float4* Mr = ch.row4(Ml);
+#pragma unroll
+    for (int q = 0; q < NVC / 4; q++) {
+      const float4 v = vec4(q), a = Mr[q];
+      s += a.x * v.x;
+      s += a.y * v.y;
+      s += a.z * v.z;
+      s += a.w * v.w;
+    }
+    s = settle(s);
+    return lane < nv ? s : 0.0f;
   }
 
   // J[r] . v for the vector last passed to put_vec (0 for r >= nr)
@@ -93,14 +108,13 @@ struct RegSolver {
     float s = 0.0f;
     if (r >= nr) return s;
     if (r < rj) {
-      const float* Jr = Jl + r * JS;
 #pragma unroll
       for (int q = 0; q < NVC / 4; q++) {
-        const float4 v = vec4(q);
-        s += Jr[4 * q] * v.x;
-        s += Jr[4 * q + 1] * v.y;
-        s += Jr[4 * q + 2] * v.z;
-        s += Jr[4 * q + 3] * v.w;
+        const float4 v = vec4(q), j = jrow4(r, q);
+        s += j.x * v.x;
+        s += j.y * v.y;
+        s += j.z * v.z;
+        s += j.w * v.w;
       }
     } else {
       gfloat* Jr = Jg(r);
@@ -151,19 +165,21 @@ struct RegSolver {
         if (s > 0 && s >= nset) break;
         if (Jaref[s] < 0.0f) act |= 1u << s;
       }
-      const float changed = sum32(act != act_prev ? 1.0f : 0.0f);
-      if (fact_valid && changed == 0.0f) {
+      const bool changed = (__ballot(act != act_prev) & team_lanes<kRegTeam>()) != 0;
+      if (fact_valid && !changed) {
         Mgrad = ch.solve(grad);
         return gd;
       }
       act_prev = act;
       fact_valid = true;
-      const int ln = opaque(lane);
-      gfloat* Mc = opaque(M) + (ln < nv ? ln : 0);
+      const float4* Mr = ch.row4(Ml);
 #pragma unroll
-      for (int j = 0; j < NVC; j++) {
-        const float v = Mc[(j < nv ? j : 0) * nv];
-        ch.h[j] = (ln < nv && j < nv) ? v : (j == ln ? 1.0f : 0.0f);
+      for (int q = 0; q < NVC / 4; q++) {
+        const float4 v = Mr[q];
+        ch.h[4 * q] = v.x;
+        ch.h[4 * q + 1] = v.y;
+        ch.h[4 * q + 2] = v.z;
+        ch.h[4 * q + 3] = v.w;
       }
       wave_fence();
 #pragma unroll
@@ -176,10 +192,15 @@ struct RegSolver {
       for (int r = 0; r < nl; r++) {
         const float dr = fbuf[r];
         if (dr == 0.0f) continue;
-        const float* Jr = Jl + r * JS;
-        const float a = lane < NVC ? dr * Jr[lane] : 0.0f;
+        const float a = lane < NVC ? dr * Jl[r * JS + lane] : 0.0f;
 #pragma unroll
-        for (int j = 0; j < NVC; j++) ch.h[j] = fmaf(a, Jr[j], ch.h[j]);
+        for (int q = 0; q < NVC / 4; q++) {
+          const float4 j = jrow4(r, q);
+          ch.h[4 * q] = fmaf(a, j.x, ch.h[4 * q]);
+          ch.h[4 * q + 1] = fmaf(a, j.y, ch.h[4 * q + 1]);
+          ch.h[4 * q + 2] = fmaf(a, j.z, ch.h[4 * q + 2]);
+          ch.h[4 * q + 3] = fmaf(a, j.w, ch.h[4 * q + 3]);
+        }
       }
       const int c = lane < nv ? lane : 0;
       for (int r = nl; r < nr; r++) {
@@ -191,11 +212,8 @@ struct RegSolver {
         for (int j = 0; j < NVC; j++) ch.h[j] = fmaf(a, j < nv ? Jr[j < nv ? j : 0] : 0.0f, ch.h[j]);
       }
       ch.factor();
-    } else if (!fact_valid) {
-      // CG preconditions with the factor of M, fixed during the solve
-      ch.load_lower(d.qLDd + (size_t)w * nv * nv, nv, blk);
-      fact_valid = true;
     }
+    // (CG preconditions with the factor of M, in ch from the start)
     Mgrad = ch.solve(grad);
     return gd;
   }
@@ -211,7 +229,8 @@ struct RegSolver {
         b += p.b;
         c += p.c;
       }
-    return V3f{sum32(a), sum32(b), sum32(c)};
+    sum32_pair(&a, &b);
+    return V3f{a, b, sum32(c)};
   }
 
   // solver.py:339-664
@@ -226,7 +245,8 @@ struct RegSolver {
         pb += q1[s];
         pc += 2.0f * q2[s];
       }
-    const V3f p0 = V3f{g0 + sum32(pa), g1 + sum32(pb), 2.0f * g2 + sum32(pc)};
+    sum32_pair(&pa, &pb);
+    const V3f p0 = V3f{g0 + pa, g1 + pb, 2.0f * g2 + sum32(pc)};
     float lo_alpha = -safe_div(p0.b, p0.c);
     V3f lo = eval_pt(g0, g1, g2, lo_alpha);
     {
@@ -265,9 +285,13 @@ struct RegSolver {
         }
       }
       V3f ln = eval_pt(g0, g1, g2, la), hn = eval_pt(g0, g1, g2, ha), mn = eval_pt(g0, g1, g2, ma);
-      ln = V3f{ln.a + sum32(s0), ln.b + sum32(s1), ln.c + sum32(s2)};
-      hn = V3f{hn.a + sum32(s3), hn.b + sum32(s4), hn.c + sum32(s5)};
-      mn = V3f{mn.a + sum32(s6), mn.b + sum32(s7), mn.c + sum32(s8)};
+      sum32_pair(&s0, &s1);
+      sum32_pair(&s2, &s3);
+      sum32_pair(&s4, &s5);
+      sum32_pair(&s6, &s7);
+      ln = V3f{ln.a + s0, ln.b + s1, ln.c + s2};
+      hn = V3f{hn.a + s3, hn.b + s4, hn.c + s5};
+      mn = V3f{mn.a + s6, mn.b + s7, mn.c + sum32(s8)};
       bool sl = false, sh = false;
       if (in_bracket(lo, ln)) { lo = ln; lo_alpha = la; sl = true; }
       if (in_bracket(lo, mn)) { lo = mn; lo_alpha = ma; sl = true; }
@@ -298,7 +322,8 @@ struct RegSolver {
           s1 += q1[s];
           s2 += q2[s];
         }
-      const float t0 = g0 + sum32(s0), t1 = g1 + sum32(s1), t2 = g2 + sum32(s2);
+      sum32_pair(&s0, &s1);
+      const float t0 = g0 + s0, t1 = g1 + s1, t2 = g2 + sum32(s2);
       const float c = a * a * t2 + a * t1 + t0;
       if (lane == 0) {
         d.efc_cost_candidate[w * m.nlsp + k] = c;
@@ -322,15 +347,15 @@ struct RegSolver {
 #pragma unroll
     for (int s = 0; s < RS; s++) {
       if (s > 0 && s >= nset) break;
-      const float v = jrow_dot(row(s));
+      const float v = settle(jrow_dot(row(s)));
       const float jar = Jaref[s], dd = D[s];
       jv[s] = v;
       q0[s] = 0.5f * jar * jar * dd;
       q1[s] = v * jar * dd;
       q2[s] = 0.5f * v * v * dd;
     }
-    const float g0 = sum32(lane < nv ? gauss / (float)nv : 0.0f);
-    const float g1 = sum32(search * (Ma - qs));
+    float g0 = lane < nv ? gauss / (float)nv : 0.0f, g1 = search * (Ma - qs);
+    sum32_pair(&g0, &g1);
     const float g2 = sum32(0.5f * search * mv);
     const float alpha = m.opt.ls_parallel ? linesearch_parallel(g0, g1, g2)
                                           : linesearch_iterative(g0, g1, g2, search_dot, prev_alpha);
@@ -343,17 +368,24 @@ struct RegSolver {
   }
 };
 
-// Solves world t.world (at most 32 RS rows) with the register solver.
-template <int NVC, int RS>
-MJH_DEV void solve_reg_nv(const mjhModel& m, const mjhData& d, float* lds, int rj, const Team<kRegTeam>& t) {
+// Solves world t.world with the register solver; returns false when it has
+// more than 32 RS rows.  kStep: all that a fused step does with the mass
+// matrix around the solve too -- its factor qLD, qacc_smooth before, the
+// integrator after -- on the one staged copy of M, the factor and the forces
+// passing on in registers (a world with too many rows gets what comes before).
+template <int NVC, int RS, bool kStep>
+MJH_DEV bool solve_reg_nv(const mjhModel& m, const mjhData& d, float* lds, int rj, const Team<kRegTeam>& t) {
   const int w = t.world, nv = m.nv;
-  const int radr = d.world_efc[2 * w], nr = d.world_efc[2 * w + 1];
+  const int radr = d.world_efc[2 * w], nr = d.njmax == 0 ? 0 : d.world_efc[2 * w + 1];
+  if (!kStep && nr > 32 * RS) return false;
   RegSolver<NVC, RS> s{m, d, w, nv, radr, nr, t.lane, rj};
   s.vbuf = lds;
   s.ch.lane = t.lane;
   s.ch.cbuf = lds + 32;
   s.fbuf = lds + 64;
-  s.Jl = lds + 64 + kRegRows;
+  float* const Ml = lds + 64 + 32 * RS;
+  s.Ml = Ml;
+  s.Jl = Ml + NVC * s.JS;
   s.nset = nr > 32 ? (nr + 31) / 32 : 1;
   s.fact_valid = false;
   s.act_prev = 0;
@@ -365,8 +397,27 @@ MJH_DEV void solve_reg_nv(const mjhModel& m, const mjhData& d, float* lds, int r
   // stage the world's inputs (solver.py:973 warm start)
   s.qacc = dof ? d.qacc_warmstart[o + lane] : 0.0f;
   s.qs = dof ? d.qfrc_smooth[o + lane] : 0.0f;
-  s.qas = dof ? d.qacc_smooth[o + lane] : 0.0f;
-  s.M = d.qMd + o * nv;
+  stage_sym<NVC>(d.qMd + o * nv, nv, lane, Ml);
+  int beg, end;
+  tree_block(m, lane, &beg, &end);
+  if (kStep) {
+    s.ch.load_rows(Ml);
+    s.ch.factor();
+    s.ch.store_rows(d.qLDd + o * nv, nv, beg, end, s.Jl, true);
+    s.ch.divide_diag(s.Jl, nv);
+    s.qas = s.ch.solve(s.qs);
+    if (dof) d.qacc_smooth[o + lane] = s.qas;
+    if (nr > 32 * RS) return false;
+  } else {
+    s.qas = dof ? d.qacc_smooth[o + lane] : 0.0f;
+    if (m.opt.solver == mjhSOL_CG) s.ch.load_lower(d.qLDd + o * nv, nv, beg, s.Jl);
+  }
+  if (kStep && d.njmax == 0) {  // forward.py:676-677
+    if (dof) d.qacc[o + lane] = s.qas;
+    integrate_reg<NVC>(m, d, m.opt.integrator == mjhINT_EULER, s.qas,
+                       dof ? s.qs + d.qfrc_constraint[o + lane] : 0.0f, s.ch.cbuf, Ml, beg, end, false, t);
+    return true;
+  }
   float aref[RS];
 #pragma unroll
   for (int k = 0; k < RS; k++) {
@@ -380,13 +431,6 @@ MJH_DEV void solve_reg_nv(const mjhModel& m, const mjhData& d, float* lds, int r
   // rows [0, nst), lanes over columns; padding columns [nv, NVC) zero
   if (lane < NVC)
     for (int r = 0; r < nst; r++) s.Jl[r * s.JS + lane] = dof ? s.Jg(r)[lane] : 0.0f;
-  if (m.opt.solver == mjhSOL_CG) {
-    // first dof of the lane's kinematic-tree block of qLD (io.py:150-162)
-    s.blk = lane;
-    for_each_tree_block(m, [&](int dof0, int n) {
-      if (lane >= dof0 && lane < dof0 + n) s.blk = dof0;
-    });
-  }
   // _create_context (solver.py:26-72)
   s.put_vec(s.qacc);
 #pragma unroll
@@ -470,21 +514,29 @@ MJH_DEV void solve_reg_nv(const mjhModel& m, const mjhData& d, float* lds, int r
     d.efc_done[w] = done;
     d.efc_solver_niter[w] = 0;
   }
+  if (kStep)
+    integrate_reg<NVC>(m, d, m.opt.integrator == mjhINT_EULER, s.qacc, s.qs + s.qc, s.ch.cbuf, Ml, beg, end, false, t);
+  return true;
 }
 
-// The register solver for world t.world with RS row sets: returns false
-// (and leaves the world untouched) when its rows exceed 32 RS.  The solve
-// launches take RS = 2 (64 rows, the register budget of two wavefronts per
-// SIMD); a tail launch takes the larger worlds with RS = kRegSets.
-template <int RS>
+// The register solver for world t.world with RS row sets (see solve_reg_nv):
+// false when its rows exceed 32 RS.  The solve launches take RS = 2 (64 rows),
+// the big-world launch RS = kRegSets.
+template <int RS, bool kStep>
 MJH_DEV bool solve_reg(const mjhModel& m, const mjhData& d, float* lds, int rj, const Team<kRegTeam>& t) {
   if (!t.valid) return true;
-  if (d.world_efc[2 * t.world + 1] > 32 * RS) return false;
-  with_nvc(m.nv, [&](auto nvc) {
-    solve_reg_nv<decltype(nvc)::value, RS>(m, d, lds, rj, t);
-    return 0;
+  if (kStep && m.opt.is_sparse) {  // MuJoCo's L'DL factor of the sparse qM
+    factor_sparse(m, WPTR(d.qM, t.world, m.nM), WPTR(d.qLD, t.world, m.nM), WPTR(d.qLDiagInv, t.world, m.nv), lds, t);
+    wave_fence();
+  }
+  const bool solved = with_nvc(m.nv, [&](auto nvc) {
+    return solve_reg_nv<decltype(nvc)::value, RS, kStep>(m, d, lds, rj, t);
   });
-  return true;
+  if (kStep && solved && m.opt.is_sparse && m.opt.integrator == mjhINT_EULER && !advances_with_qacc(m)) {
+    wave_fence();
+    euler_sparse_outputs(m, d, lds, t);
+  }
+  return solved;
 }
 
 }  // namespace mjh

@@ -71,16 +71,11 @@ STAGE(StQaccSmooth, if (t.valid) for (int i = t.lane; i < m.nv; i += T) d.qacc[t
 // else the LDS solver; false when the world is left for the tail.
 template <int T>
 MJH_DEV bool solve_team(const mjhModel& m, const mjhData& d, float* l, const Team<T>& t, const Tune& tune) {
-  if constexpr (T == kRegTeam) return solve_reg<2>(m, d, l, tune.rj, t);
+  if constexpr (T == kRegTeam) return solve_reg<2, false>(m, d, l, tune.rj, t);
   else return solve_lds(m, d, l, tune.rmax, tune.rj, tune.wide != 0, t);
 }
-// Worlds the 32-lane solve launches leave to the big-world launch: more
-// rows than two row sets hold, at most kRegRows.
-MJH_DEV bool big_world(const mjhData& d, int w) {
-  if (d.njmax == 0) return false;
-  const int nr = d.world_efc[2 * w + 1];
-  return nr > 2 * kRegTeam && nr <= kRegRows;
-}
+// Worlds the 32-lane solve launches leave to the big-world launch.
+MJH_DEV bool big_world(const mjhData& d, int w) { return d.njmax != 0 && big_rows(d.world_efc[2 * w + 1]); }
 template <int T>
 MJH_DEV bool left_to_big(const mjhData& d, const Team<T>& t) {
   if constexpr (T == kRegTeam) return t.valid && big_world(d, t.world);
@@ -95,20 +90,16 @@ STAGE(StSolveTeam, if (left_to_big(d, t)) return;
 template <bool step>
 struct StBigWorlds {
   template <int T>
-  MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<T>& t, const Tune& tune) const {
+  MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<T>& place, const Tune& tune) const {
     static_assert(T == kRegTeam, "big worlds run on 32-lane teams");
+    Team<T> t = place;
+    // (without constraint rows built, the map says nothing)
+    if (const unsigned* map = (m.opt.disableflags & mjhDSBL_CONSTRAINT) ? nullptr : big_map(d)) {
+      t.world = big_map_world(d, map, place.world);
+      t.valid = place.valid && t.world >= 0 && t.world < d.nworld;
+    }
     if (!t.valid || !big_world(d, t.world)) return;
-    if (step) {
-      factor_m(m, d, l, t);
-      sync();
-      fwd_acceleration_solve(m, d, l, t);
-    }
-    solve_reg<kRegSets>(m, d, l, tune.rj, t);
-    sync();
-    if (step) {
-      if (m.opt.integrator == mjhINT_EULER) euler(m, d, l, t);
-      else implicit(m, d, l, t);
-    }
+    solve_reg<kRegSets, step>(m, d, l, tune.rj, t);
   }
 };
 
@@ -202,21 +193,10 @@ struct StFusedForward {
 struct StFusedSolveIntegrate {
   template <int T>
   MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<T>& t, const Tune& tune) const {
+    static_assert(T == kRegTeam, "64-lane teams take the three launches below");
     if (left_to_big(d, t)) return;  // StBigWorlds<true> steps it
-    factor_m(m, d, l, t);
-    sync();
-    fwd_acceleration_solve(m, d, l, t);
-    if (d.njmax == 0) {
-      if (t.valid)
-        for (int i = t.lane; i < m.nv; i += T) d.qacc[t.world * m.nv + i] = d.qacc_smooth[t.world * m.nv + i];
-      sync();
-    } else if (!solve_team(m, d, l, t, tune)) {
-      if (t.lane == 0) d.world_flags[t.world] |= kFlagDeferred;
-      return;  // solved and integrated by the tail launch
-    }
-    sync();
-    if (m.opt.integrator == mjhINT_EULER) euler(m, d, l, t);
-    else implicit(m, d, l, t);
+    // a world past the solver's rows is solved and integrated by the tail launch
+    if (!solve_reg<2, true>(m, d, l, tune.rj, t) && t.lane == 0) d.world_flags[t.world] |= kFlagDeferred;
   }
 };
 
@@ -267,14 +247,17 @@ __global__ void __launch_bounds__(64) k_stage(mjhModel m, mjhData d, int lds_per
   S()(m, d, smem + t.slot * lds_per_world, t, tune);
 }
 
-// counter reset without memset nodes (capture-safe):
-// which bit 0: ncollision + ncon, bit 1: nefc
+// counter reset without memset nodes (capture-safe), by one workgroup:
+// which bit 0: ncollision + ncon, bit 1: nefc and the big-world map
 MJH_DEV void reset_counters(const mjhData& d, int which) {
-  if (which & 1) {
+  if ((which & 1) && threadIdx.x == 0) {
     d.ncollision[0] = 0;
     d.ncon[0] = 0;
   }
-  if (which & 2) d.nefc[0] = 0;
+  if (which & 2) {
+    if (threadIdx.x == 0) d.nefc[0] = 0;
+    clear_big_map(d, threadIdx.x, blockDim.x);
+  }
 }
 
 // ---- heterogeneous batches: several (model, data) groups, each with its
