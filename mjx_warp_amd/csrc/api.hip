@@ -306,7 +306,7 @@ constexpr int kLdsRowsMin = 256, kLdsRowsMax = 1024;
 // defaults, MJH_SOLVER_WIDE=1 / 0 puts the Hessian of any 64-lane model in
 // efc_h / in LDS (where it fits).
 Tune tune_for(const mjhModel& m, bool reg) {
-  Tune t{64, 0, 0};
+  Tune t{64, 0, 0, 0, 0};
   if (reg) {
     // as many Jacobian rows as leave a CU twelve workgroups (three wavefronts
     // per SIMD, what the registers allow), at least the nvc the solver's
@@ -345,6 +345,7 @@ Tune tune_for(const mjhModel& m, bool reg) {
   t.tail_rows = !reg && lds_solver_floats(m.nv, kLdsRowsMax, 0, t.wide != 0) <= (int)(lds_cap() / sizeof(float))
                     ? kLdsRowsMax
                     : 0;
+  t.resident = fwd_resident(m, reg ? kRegTeam : kTeam, (int)(lds_cap() / sizeof(float)));
   return t;
 }
 Tune tune_for(const mjhModel& m) { return tune_for(m, reg_path(m)); }
@@ -373,7 +374,10 @@ int lds_forward(const mjhModel& m, bool reg) {
   a = a > b ? a : b;
   a = a > c ? a : c;
   a = a > k ? a : k;
-  return a > g ? a : g;
+  a = a > g ? a : g;
+  const int team = reg ? kRegTeam : kTeam;
+  const int r = fwd_resident(m, team, (int)(lds_cap() / sizeof(float))) ? fwd_lds(m, team).total : 0;
+  return a > r ? a : r;
 }
 int lds_forward(const mjhModel& m) { return lds_forward(m, reg_path(m)); }
 // the 64-lane fused step (forward, LDS solver, integrator in one launch)
@@ -636,7 +640,10 @@ int do_step_fused(const mjhModel& m, const mjhData& d, hipStream_t s) {
   if (d.step_desc && d.nworld > 0) return do_step_fused_desc(m, d, s);
   TRY(reset(d, s, (m.opt.disableflags & mjhDSBL_CONSTRAINT) ? 1 : 3));
   if (reg_path(m)) {
-    TRY((launch_team<StFusedForward, kRegTeam>(m, d, s, lds_forward_reg(m), "step_fused_forward")));
+    // (the resident form reads the model too widely for a kernel argument)
+    Tune tf = tune_for(m);
+    tf.resident = 0;
+    TRY((launch_team<StFusedForward, kRegTeam>(m, d, s, lds_forward_reg(m), "step_fused_forward", &tf)));
     const Tune tt = tune_tail_reg(m);
     TRY(beside(
         s,

@@ -528,13 +528,27 @@ MJH_DEV void closest_segment_to_segment_points(V3 a0, V3 a1, V3 b0, V3 b1, V3* r
   }
 }
 
+// The geoms' poses as the narrowphase reads them: from Data, or from the
+// records of forward_lds.hpp (position and rotation first).
+struct GeomPoses {
+  const float *gxpos, *gxmat;
+  MJH_DEV V3 pos(int g) const { return ld3(gxpos + 3 * g); }
+  MJH_DEV M33 mat(int g) const { return ld9(gxmat + 9 * g); }
+};
+struct GeomRecords {
+  const float* rec;
+  static constexpr int stride = 15;
+  MJH_DEV V3 pos(int g) const { return ld3(rec + stride * g); }
+  MJH_DEV M33 mat(int g) const { return ld9(rec + stride * g + 3); }
+};
+
 // collision_primitive.py:235-268 dispatch on (type1 <= type2)
-MJH_DEV void narrowphase_pair(const mjhModel& m, const float* gxpos, const float* gxmat, int g1, int g2,
-                              ContactSink& s) {
+template <class Poses>
+MJH_DEV void narrowphase_pair(const mjhModel& m, const Poses& poses, int g1, int g2, ContactSink& s) {
   const int t1 = m.geom_type[g1], t2 = m.geom_type[g2];
   const float margin = fmaxf(m.geom_margin[g1], m.geom_margin[g2]);
-  const V3 p1 = ld3(gxpos + 3 * g1), p2 = ld3(gxpos + 3 * g2);
-  const M33 r1 = ld9(gxmat + 9 * g1), r2 = ld9(gxmat + 9 * g2);
+  const V3 p1 = poses.pos(g1), p2 = poses.pos(g2);
+  const M33 r1 = poses.mat(g1), r2 = poses.mat(g2);
   const float* s1 = m.geom_size + 3 * g1;
   const float* s2 = m.geom_size + 3 * g2;
   s.g1 = g1;
@@ -586,6 +600,10 @@ MJH_DEV void narrowphase_pair(const mjhModel& m, const float* gxpos, const float
     sphere_sphere(pt1, s1[0], pt2, s2[0], margin, s);
   }
   // sphere-capsule and other pairs produce no contacts in the reference
+}
+MJH_DEV void narrowphase_pair(const mjhModel& m, const float* gxpos, const float* gxmat, int g1, int g2,
+                              ContactSink& s) {
+  narrowphase_pair(m, GeomPoses{gxpos, gxmat}, g1, g2, s);
 }
 
 // collision_driver.py:62-65: pairs are ordered by geom type

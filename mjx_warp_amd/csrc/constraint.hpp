@@ -116,16 +116,17 @@ MJH_DEV int big_map_world(const mjhData& d, const unsigned* map, int i) {
 // The rows of one world into the block [base, base + total) of the pool
 // (reserved by the caller; total counts nlim limit rows first): limit rows
 // in joint order, then four rows per active contact in contact order, as
-// many as the block and the pool hold.
-template <int TEAM>
+// many as the block and the pool hold.  qpos, qvel, cdof and sc (subtree_com)
+// of the world lie in global memory or LDS; moves(b, i): whether dof i moves
+// body b; contacts are taken CHUNK at a time (29 floats of LDS each).
+template <int TEAM, int CHUNK, class Moves>
 MJH_DEV void make_constraint_rows(const mjhModel& m, const mjhData& d, float* lds, const Team<TEAM>& t, int base,
-                                  int total, int nlim) {
+                                  int total, int nlim, const float* qpos, const float* qvel, const float* cdof,
+                                  const float* sc, Moves moves) {
   const int w = t.world, nv = m.nv;
   const bool refsafe = !(m.opt.disableflags & mjhDSBL_REFSAFE);
   const bool do_limit = !(m.opt.disableflags & mjhDSBL_LIMIT) && m.nlimited > 0;
   const bool do_contact = !(m.opt.disableflags & mjhDSBL_CONTACT) && m.opt.cone == mjhCONE_PYRAMIDAL;
-  const float* qpos = WPTR(d.qpos, w, m.nq);
-  const float* qvel = WPTR(d.qvel, w, nv);
   int cadr = 0, ncon = 0;
   if (t.valid && do_contact) {
     cadr = d.world_con[2 * w];
@@ -166,24 +167,22 @@ MJH_DEV void make_constraint_rows(const mjhModel& m, const mjhData& d, float* ld
       }
       k0 += tot;
     }
-  // contact rows (constraint.py:144-210), in chunks of TEAM contacts: the
+  // contact rows (constraint.py:144-210), in chunks of CHUNK contacts: the
   // per-contact scalars are gathered with lanes over contacts, the Jacobian
   // rows are built one contact at a time with lanes over dofs, and the
   // impedance / reference terms are computed with lanes over rows.  A
   // contact's four rows are written only if all four fit.
   int* lci = (int*)lds;
-  int* lrr = lci + TEAM;
-  int* lb = lrr + TEAM;
-  int* lact = lb + 2 * TEAM;
-  float* lf = (float*)(lact + TEAM);
-  float* ljq = lf + 20 * TEAM;
-  const float* cdof = WPTR(d.cdof, w, nv * 6);
-  const float* sc = WPTR(d.subtree_com, w, m.nbody * 3);
+  int* lrr = lci + CHUNK;
+  int* lb = lrr + CHUNK;
+  int* lact = lb + 2 * CHUNK;
+  float* lf = (float*)(lact + CHUNK);
+  float* ljq = lf + 20 * CHUNK;
   int rrun = nlim;  // rows of this world so far
-  for (int c0 = 0; c0 < ncon; c0 += TEAM) {
+  for (int c0 = 0; c0 < ncon; c0 += CHUNK) {
     const int c = c0 + t.lane;
     bool act = false;
-    if (c < ncon) {
+    if (t.lane < CHUNK && c < ncon) {
       const int ci = cadr + c;
       const float pos = d.contact_dist[ci] - d.contact_includemargin[ci];
       act = d.contact_dim[ci] == 3 && pos < 0.0f;
@@ -232,8 +231,8 @@ MJH_DEV void make_constraint_rows(const mjhModel& m, const mjhData& d, float* ld
         const V3 rot = V3{cd.v[0], cd.v[1], cd.v[2]}, lin = V3{cd.v[3], cd.v[4], cd.v[5]};
         V3 jac1 = lin + cross(rot, off1);
         V3 jac2 = lin + cross(rot, off2);
-        if (!m.body_dof_tree[b1 * nv + i]) jac1 = V3{0.f, 0.f, 0.f};
-        if (!m.body_dof_tree[b2 * nv + i]) jac2 = V3{0.f, 0.f, 0.f};
+        if (!moves(b1, i)) jac1 = V3{0.f, 0.f, 0.f};
+        if (!moves(b2, i)) jac2 = V3{0.f, 0.f, 0.f};
         const V3 jd = jac2 - jac1;
         const float d0 = dot(n, jd), d1 = dot(t1, jd), d2 = dot(t2, jd);
         const float J0 = d0 + d1 * fr0;
@@ -269,6 +268,16 @@ MJH_DEV void make_constraint_rows(const mjhModel& m, const mjhData& d, float* ld
     sync();
     rrun += 4 * nact;
   }
+}
+
+// ... on the world's fields in global memory
+template <int TEAM>
+MJH_DEV void make_constraint_rows(const mjhModel& m, const mjhData& d, float* lds, const Team<TEAM>& t, int base,
+                                  int total, int nlim) {
+  const int w = t.world, nv = m.nv;
+  make_constraint_rows<TEAM, TEAM>(m, d, lds, t, base, total, nlim, WPTR(d.qpos, w, m.nq), WPTR(d.qvel, w, nv),
+                                   WPTR(d.cdof, w, nv * 6), WPTR(d.subtree_com, w, m.nbody * 3),
+                                   [&](int b, int i) { return m.body_dof_tree[b * nv + i]; });
 }
 
 // constraint.py:213-240 make_constraint (nefc is reset by the caller):

@@ -59,6 +59,25 @@ MJH_DEV void fwd_velocity(const mjhModel& m, const mjhData& d, float* lds, const
   rne(m, d, lds, t);
 }
 
+// forward.py:503-560: one actuator's force
+MJH_DEV float actuator_force(const mjhModel& m, int a, float length, float velocity, float ctrl) {
+  const bool noclamp = m.opt.disableflags & mjhDSBL_CLAMPCTRL;
+  const float* g = m.actuator_gainprm + 10 * a;
+  const float* b = m.actuator_biasprm + 10 * a;
+  float gain = g[0];
+  gain += g[1] * length;
+  gain += g[2] * velocity;
+  float bias = b[0];
+  bias += b[1] * length;
+  bias += b[2] * velocity;
+  float c = ctrl;
+  if (m.actuator_ctrllimited[a] && !noclamp)
+    c = fminf(fmaxf(c, m.actuator_ctrlrange[2 * a]), m.actuator_ctrlrange[2 * a + 1]);
+  // actuator forcerange is read but never applied by the reference
+  // (forward.py:539-541)
+  return gain * c + bias;
+}
+
 // forward.py:503-641 fwd_actuation
 template <int TEAM>
 MJH_DEV void fwd_actuation(const mjhModel& m, const mjhData& d, const Team<TEAM>& t) {
@@ -78,22 +97,8 @@ MJH_DEV void fwd_actuation(const mjhModel& m, const mjhData& d, const Team<TEAM>
     const float* length = WPTR(d.actuator_length, w, nu);
     const float* velocity = WPTR(d.actuator_velocity, w, nu);
     const float* ctrl = WPTR(d.ctrl, w, nu);
-    const bool noclamp = m.opt.disableflags & mjhDSBL_CLAMPCTRL;
     for (int a = t.lane; a < nu; a += TEAM) {
-      const float* g = m.actuator_gainprm + 10 * a;
-      const float* b = m.actuator_biasprm + 10 * a;
-      float gain = g[0];
-      gain += g[1] * length[a];
-      gain += g[2] * velocity[a];
-      float bias = b[0];
-      bias += b[1] * length[a];
-      bias += b[2] * velocity[a];
-      float c = ctrl[a];
-      if (m.actuator_ctrllimited[a] && !noclamp)
-        c = fminf(fmaxf(c, m.actuator_ctrlrange[2 * a]), m.actuator_ctrlrange[2 * a + 1]);
-      // actuator forcerange is read but never applied by the reference
-      // (forward.py:539-541)
-      force[a] = gain * c + bias;
+      force[a] = actuator_force(m, a, length[a], velocity[a], ctrl[a]);
     }
   }
   sync();

@@ -138,6 +138,55 @@ MJH_DEV void kinematics(const mjhModel& m, const mjhData& d, float* lds, const T
 }
 
 // ---------------------------------------------------------------------------
+// smooth.py:190-215: the com-frame inertia of a body (mat: its inertia frame,
+// dif: its centre off the tree's centre of mass) into r[10]
+MJH_DEV void body_cinert(float* r, const M33& mat, V3 inert, float mass, V3 dif) {
+  // mat * diag(inert) * mat'
+  float tmp[3][3];
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      tmp[i][j] = mat.m[3 * i] * inert.x * mat.m[3 * j] + mat.m[3 * i + 1] * inert.y * mat.m[3 * j + 1] +
+                  mat.m[3 * i + 2] * inert.z * mat.m[3 * j + 2];
+  r[0] = tmp[0][0] + mass * (dif.y * dif.y + dif.z * dif.z);
+  r[1] = tmp[1][1] + mass * (dif.x * dif.x + dif.z * dif.z);
+  r[2] = tmp[2][2] + mass * (dif.x * dif.x + dif.y * dif.y);
+  r[3] = tmp[0][1] - mass * dif.x * dif.y;
+  r[4] = tmp[0][2] - mass * dif.x * dif.z;
+  r[5] = tmp[1][2] - mass * dif.y * dif.z;
+  r[6] = mass * dif.x;
+  r[7] = mass * dif.y;
+  r[8] = mass * dif.z;
+  r[9] = mass;
+}
+
+// smooth.py:217-235: the motion axes of a joint from its axis, its body's
+// rotation xmat and its anchor's offset to the tree's centre of mass
+MJH_DEV void joint_cdof(float* cdof, int jt, V3 axis, const float* xmat, V3 offset) {
+  if (jt == mjhJNT_FREE || jt == mjhJNT_BALL) {
+    const M33 xm = ld9(xmat);
+    float* c = cdof;
+    if (jt == mjhJNT_FREE) {
+      for (int i = 0; i < 3; i++, c += 6) {
+        for (int k = 0; k < 6; k++) c[k] = 0.0f;
+        c[3 + i] = 1.0f;
+      }
+    }
+    for (int i = 0; i < 3; i++, c += 6) {
+      const V3 ax = mcol(xm, i);  // row i of xmat' = column i of xmat
+      st3(c, ax);
+      st3(c + 3, cross(ax, offset));
+    }
+  } else if (jt == mjhJNT_SLIDE) {
+    st3(cdof, V3{0.f, 0.f, 0.f});
+    st3(cdof + 3, axis);
+  } else {
+    st3(cdof, axis);
+    st3(cdof + 3, cross(axis, offset));
+  }
+}
+
 // smooth.py:148-245 com_pos
 // lds: 3 * nbody floats; holds the subtree sums / centres of mass
 template <int TEAM>
@@ -168,29 +217,8 @@ MJH_DEV void com_pos(const mjhModel& m, const mjhData& d, float* lds, const Team
     const float* ximat = WPTR(d.ximat, w, nbody * 9);
     float* cinert = WPTR(d.cinert, w, nbody * 10);
     for (int b = t.lane; b < nbody; b += TEAM) {
-      const M33 mat = ld9(ximat + 9 * b);
-      const V3 inert = ld3(m.body_inertia + 3 * b);
-      const float mass = m.body_mass[b];
-      const V3 dif = ld3(xipos + 3 * b) - ld3(sc + 3 * m.body_rootid[b]);
-      // mat * diag(inert) * mat'
-      float tmp[3][3];
-#pragma unroll
-      for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++)
-          tmp[i][j] = mat.m[3 * i] * inert.x * mat.m[3 * j] + mat.m[3 * i + 1] * inert.y * mat.m[3 * j + 1] +
-                      mat.m[3 * i + 2] * inert.z * mat.m[3 * j + 2];
-      float* r = cinert + 10 * b;
-      r[0] = tmp[0][0] + mass * (dif.y * dif.y + dif.z * dif.z);
-      r[1] = tmp[1][1] + mass * (dif.x * dif.x + dif.z * dif.z);
-      r[2] = tmp[2][2] + mass * (dif.x * dif.x + dif.y * dif.y);
-      r[3] = tmp[0][1] - mass * dif.x * dif.y;
-      r[4] = tmp[0][2] - mass * dif.x * dif.z;
-      r[5] = tmp[1][2] - mass * dif.y * dif.z;
-      r[6] = mass * dif.x;
-      r[7] = mass * dif.y;
-      r[8] = mass * dif.z;
-      r[9] = mass;
+      body_cinert(cinert + 10 * b, ld9(ximat + 9 * b), ld3(m.body_inertia + 3 * b), m.body_mass[b],
+                  ld3(xipos + 3 * b) - ld3(sc + 3 * m.body_rootid[b]));
     }
     const float* xaxis = WPTR(d.xaxis, w, m.njnt * 3);
     const float* xanchor = WPTR(d.xanchor, w, m.njnt * 3);
@@ -198,37 +226,8 @@ MJH_DEV void com_pos(const mjhModel& m, const mjhData& d, float* lds, const Team
     float* cdof = WPTR(d.cdof, w, m.nv * 6);
     for (int j = t.lane; j < m.njnt; j += TEAM) {
       const int b = m.jnt_bodyid[j];
-      const int da = m.jnt_dofadr[j];
-      const int jt = m.jnt_type[j];
-      const V3 axis = ld3(xaxis + 3 * j);
-      const M33 xm = ld9(xmat + 9 * b);
-      const V3 offset = ld3(sc + 3 * m.body_rootid[b]) - ld3(xanchor + 3 * j);
-      if (jt == mjhJNT_FREE || jt == mjhJNT_BALL) {
-        int r0 = da;
-        if (jt == mjhJNT_FREE) {
-          for (int i = 0; i < 3; i++) {
-            float* c = cdof + 6 * (da + i);
-            for (int k = 0; k < 6; k++) c[k] = 0.0f;
-            c[3 + i] = 1.0f;
-          }
-          r0 = da + 3;
-        }
-        for (int i = 0; i < 3; i++) {
-          const V3 ax = mcol(xm, i);  // row i of xmat' = column i of xmat
-          const V3 lin = cross(ax, offset);
-          float* c = cdof + 6 * (r0 + i);
-          st3(c, ax);
-          st3(c + 3, lin);
-        }
-      } else if (jt == mjhJNT_SLIDE) {
-        float* c = cdof + 6 * da;
-        st3(c, V3{0.f, 0.f, 0.f});
-        st3(c + 3, axis);
-      } else {
-        float* c = cdof + 6 * da;
-        st3(c, axis);
-        st3(c + 3, cross(axis, offset));
-      }
+      joint_cdof(cdof + 6 * m.jnt_dofadr[j], m.jnt_type[j], ld3(xaxis + 3 * j), xmat + 9 * b,
+                 ld3(sc + 3 * m.body_rootid[b]) - ld3(xanchor + 3 * j));
     }
   }
   sync();
@@ -587,6 +586,15 @@ MJH_DEV void factor_m(const mjhModel& m, const mjhData& d, float* lds, const Tea
 }
 
 // ---------------------------------------------------------------------------
+// smooth.py:430-445: a body's inertial and gyroscopic force
+MJH_DEV S6 body_force(const float* ci, const S6& acc, const S6& v) {
+  S6 f = inert_vec(ci, acc);
+  const S6 g = motion_cross_force(v, inert_vec(ci, v));
+#pragma unroll
+  for (int c = 0; c < 6; c++) f.v[c] += g.v[c];
+  return f;
+}
+
 // smooth.py:398-466 rne
 // lds: lds_velocity_floats; holds the body accelerations and forces
 template <int TEAM>
@@ -630,13 +638,7 @@ MJH_DEV void rne(const mjhModel& m, const mjhData& d, float* lds, const Team<TEA
     const float* cinert = WPTR(d.cinert, w, nbody * 10);
     const float* cvel = WPTR(d.cvel, w, nbody * 6);
     for (int b = t.lane; b < nbody; b += TEAM) {
-      const float* ci = cinert + 10 * b;
-      S6 f = inert_vec(ci, ld6(cacc + 6 * b));
-      const S6 v = ld6(cvel + 6 * b);
-      const S6 g = motion_cross_force(v, inert_vec(ci, v));
-#pragma unroll
-      for (int c = 0; c < 6; c++) f.v[c] += g.v[c];
-      st6(cfrc + 6 * b, f);
+      st6(cfrc + 6 * b, body_force(cinert + 10 * b, ld6(cacc + 6 * b), ld6(cvel + 6 * b)));
     }
   }
   sync();
@@ -706,6 +708,39 @@ MJH_DEV void transmission(const mjhModel& m, const mjhData& d, const Team<TEAM>&
 }
 
 // ---------------------------------------------------------------------------
+// smooth.py:555-600: one joint's part of a body's velocity v and its axes'
+// derivatives; returns the next joint's first dof
+MJH_DEV int joint_velocity(S6& v, int jt, int da, const float* cdof, float* cdof_dot, const float* qvel) {
+  if (jt == mjhJNT_FREE) {
+    for (int i = 0; i < 3; i++) {
+      const S6 c = ld6(cdof + 6 * (da + i));
+#pragma unroll
+      for (int q = 0; q < 6; q++) v.v[q] += c.v[q] * qvel[da + i];
+    }
+    for (int i = 3; i < 6; i++) st6(cdof_dot + 6 * (da + i), motion_cross(v, ld6(cdof + 6 * (da + i))));
+    for (int i = 3; i < 6; i++) {
+      const S6 c = ld6(cdof + 6 * (da + i));
+#pragma unroll
+      for (int q = 0; q < 6; q++) v.v[q] += c.v[q] * qvel[da + i];
+    }
+    return da + 6;
+  }
+  if (jt == mjhJNT_BALL) {
+    for (int i = 0; i < 3; i++) st6(cdof_dot + 6 * (da + i), motion_cross(v, ld6(cdof + 6 * (da + i))));
+    for (int i = 0; i < 3; i++) {
+      const S6 c = ld6(cdof + 6 * (da + i));
+#pragma unroll
+      for (int q = 0; q < 6; q++) v.v[q] += c.v[q] * qvel[da + i];
+    }
+    return da + 3;
+  }
+  const S6 c = ld6(cdof + 6 * da);
+  st6(cdof_dot + 6 * da, motion_cross(v, c));
+#pragma unroll
+  for (int q = 0; q < 6; q++) v.v[q] += c.v[q] * qvel[da];
+  return da + 1;
+}
+
 // smooth.py:539-606 com_vel
 // lds: 6 * nbody floats; holds the body velocities
 template <int TEAM>
@@ -731,35 +766,7 @@ MJH_DEV void com_vel(const mjhModel& m, const mjhData& d, float* lds, const Team
       const int ja = m.body_jntadr[b], jn = m.body_jntnum[b];
       S6 v = ld6(cvel + 6 * pid);
       for (int j = ja; j < ja + jn; j++) {
-        const int jt = m.jnt_type[j];
-        if (jt == mjhJNT_FREE) {
-          for (int i = 0; i < 3; i++) {
-            const S6 c = ld6(cdof + 6 * (da + i));
-#pragma unroll
-            for (int q = 0; q < 6; q++) v.v[q] += c.v[q] * qvel[da + i];
-          }
-          for (int i = 3; i < 6; i++) st6(cdof_dot + 6 * (da + i), motion_cross(v, ld6(cdof + 6 * (da + i))));
-          for (int i = 3; i < 6; i++) {
-            const S6 c = ld6(cdof + 6 * (da + i));
-#pragma unroll
-            for (int q = 0; q < 6; q++) v.v[q] += c.v[q] * qvel[da + i];
-          }
-          da += 6;
-        } else if (jt == mjhJNT_BALL) {
-          for (int i = 0; i < 3; i++) st6(cdof_dot + 6 * (da + i), motion_cross(v, ld6(cdof + 6 * (da + i))));
-          for (int i = 0; i < 3; i++) {
-            const S6 c = ld6(cdof + 6 * (da + i));
-#pragma unroll
-            for (int q = 0; q < 6; q++) v.v[q] += c.v[q] * qvel[da + i];
-          }
-          da += 3;
-        } else {
-          const S6 c = ld6(cdof + 6 * da);
-          st6(cdof_dot + 6 * da, motion_cross(v, c));
-#pragma unroll
-          for (int q = 0; q < 6; q++) v.v[q] += c.v[q] * qvel[da];
-          da += 1;
-        }
+        da = joint_velocity(v, m.jnt_type[j], da, cdof, cdof_dot, qvel);
       }
       st6(cvel + 6 * b, v);
       st6(cvelw + 6 * b, v);
@@ -769,6 +776,27 @@ MJH_DEV void com_vel(const mjhModel& m, const mjhData& d, float* lds, const Team
 }
 
 // ---------------------------------------------------------------------------
+// passive.py:27-80: a joint's spring forces into spring (by dof)
+MJH_DEV void joint_spring(const mjhModel& m, int j, const float* qpos, float* spring) {
+  const float k = m.jnt_stiffness[j];
+  if (k == 0.0f) return;
+  const int da = m.jnt_dofadr[j], qa = m.jnt_qposadr[j], jt = m.jnt_type[j];
+  if (jt == mjhJNT_FREE) {
+    for (int i = 0; i < 3; i++) spring[da + i] = -k * (qpos[qa + i] - m.qpos_spring[qa + i]);
+    const V3 dif = quat_sub(ld4(qpos + qa + 3), ld4(m.qpos_spring + qa + 3));
+    spring[da + 3] = -k * dif.x;
+    spring[da + 4] = -k * dif.y;
+    spring[da + 5] = -k * dif.z;
+  } else if (jt == mjhJNT_BALL) {
+    const V3 dif = quat_sub(ld4(qpos + qa), ld4(m.qpos_spring + qa));
+    spring[da + 0] = -k * dif.x;
+    spring[da + 1] = -k * dif.y;
+    spring[da + 2] = -k * dif.z;
+  } else {
+    spring[da] = -k * (qpos[qa] - m.qpos_spring[qa]);
+  }
+}
+
 // passive.py:27-108 passive
 template <int TEAM>
 MJH_DEV void passive(const mjhModel& m, const mjhData& d, const Team<TEAM>& t) {
@@ -789,23 +817,7 @@ MJH_DEV void passive(const mjhModel& m, const mjhData& d, const Team<TEAM>& t) {
   sync();
   if (t.valid) {
     for (int j = t.lane; j < m.njnt; j += TEAM) {
-      const float k = m.jnt_stiffness[j];
-      if (k == 0.0f) continue;
-      const int da = m.jnt_dofadr[j], qa = m.jnt_qposadr[j], jt = m.jnt_type[j];
-      if (jt == mjhJNT_FREE) {
-        for (int i = 0; i < 3; i++) spring[da + i] = -k * (qpos[qa + i] - m.qpos_spring[qa + i]);
-        const V3 dif = quat_sub(ld4(qpos + qa + 3), ld4(m.qpos_spring + qa + 3));
-        spring[da + 3] = -k * dif.x;
-        spring[da + 4] = -k * dif.y;
-        spring[da + 5] = -k * dif.z;
-      } else if (jt == mjhJNT_BALL) {
-        const V3 dif = quat_sub(ld4(qpos + qa), ld4(m.qpos_spring + qa));
-        spring[da + 0] = -k * dif.x;
-        spring[da + 1] = -k * dif.y;
-        spring[da + 2] = -k * dif.z;
-      } else {
-        spring[da] = -k * (qpos[qa] - m.qpos_spring[qa]);
-      }
+      joint_spring(m, j, qpos, spring);
     }
   }
   sync();

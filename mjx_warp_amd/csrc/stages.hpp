@@ -14,6 +14,7 @@
 #include "constraint.hpp"
 #include "derivative.hpp"
 #include "forward.hpp"
+#include "forward_lds.hpp"
 #include "smooth.hpp"
 #include "solver.hpp"
 #include "solver_lds.hpp"
@@ -27,12 +28,14 @@ constexpr int kTeam = 64;
 // staged J rows; wide: the Newton Hessians of the 64-lane solvers live in
 // efc_h (global) instead of LDS, for models whose nv^2 does not fit;
 // tail_rows: the row capacity of the LDS solver in the tail launch (0: the
-// tail has only the global-memory solver)
+// tail has only the global-memory solver); resident: the fused forward
+// launch keeps the world's state in LDS (fwd_resident)
 struct Tune {
   int rmax;
   int rj;
   int wide;
   int tail_rows;
+  int resident;
 };
 
 #define STAGE(NAME, CALL)                                                                              \
@@ -177,7 +180,11 @@ struct StFusedStep {
 // groups would impose that register budget on the whole step.
 struct StFusedForward {
   template <int T>
-  MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<T>& t, const Tune&) const {
+  MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<T>& t, const Tune& tune) const {
+    if (tune.resident) {
+      forward_resident(m, d, l, t);
+      return;
+    }
     kinematics(m, d, l, t);
     com_pos(m, d, l, t);
     crb(m, d, l, t);
