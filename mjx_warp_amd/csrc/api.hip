@@ -294,17 +294,19 @@ constexpr int kLdsRowsMin = 256, kLdsRowsMax = 1024;
 // 64-lane teams.  On the 64-lane path no rows are staged (the LDS solver
 // stages a world's rows only when all of them fit, and the LDS that takes
 // costs occupancy: the three attached humanoids step 1.25x faster without
-// it); the Newton Hessian moves to efc_h (wide, factored there in LDS
-// panels) when with it in LDS next to 256 rows a CU would hold fewer than
-// five workgroups (three attached humanoids, nv 81: 1.03e6 world-steps/s
-// wide, 0.89e6 in LDS; a 40-link chain, nv 40: 2.3e6 wide, 2.75e6 in LDS);
+// it); the Newton Hessian is packed in LDS and factored from registers
+// (kHessTri) up to two rows per lane while next to 256 rows a CU holds three
+// workgroups (three attached humanoids, nv 81, step in ms, before / packed:
+// 1 world 3.9 / 2.2, 1024 worlds 4.5 / 2.2, 4096 worlds 8.2 / 5.2); past that
+// it is square in LDS or, where a CU would then hold fewer than five
+// workgroups, in efc_h (factored there in LDS panels);
 // and the row capacity fills what
 // the solver's LDS leaves before a CU would hold one workgroup fewer (a CU
 // holds lds_cap() bytes: 160 KiB on gfx950): rows cost 8 floats each, and a
 // world with more rows than the capacity is solved by the slower
 // global-memory tail.  MJH_SOLVER_RMAX / MJH_SOLVER_RJ override the
 // defaults, MJH_SOLVER_WIDE=1 / 0 puts the Hessian of any 64-lane model in
-// efc_h / in LDS (where it fits).
+// efc_h / square in LDS (where it fits).
 Tune tune_for(const mjhModel& m, bool reg) {
   Tune t{64, 0, 0, 0, 0};
   if (reg) {
@@ -319,17 +321,20 @@ Tune tune_for(const mjhModel& m, bool reg) {
     t.rmax = kLdsRowsMin;
     const int cap = (int)(lds_cap() / sizeof(float));
     const bool fits = lds_solver_floats(m.nv, kLdsRowsMin, t.rj) <= cap && lds_tail(m, false) <= cap;
-    t.wide = !fits || lds_solver_floats(m.nv, kLdsRowsMin, t.rj) > cap / 5;
+    t.hess = !fits || lds_solver_floats(m.nv, kLdsRowsMin, t.rj) > cap / 5 ? kHessGlobal : kHessSquare;
+    if (m.opt.solver == mjhSOL_NEWTON && m.nv <= kTriMax &&
+        lds_solver_floats(m.nv, kLdsRowsMin, t.rj, kHessTri) <= cap / 3)
+      t.hess = kHessTri;
     if (const char* e = std::getenv("MJH_SOLVER_WIDE")) {
-      if (std::strcmp(e, "1") == 0) t.wide = 1;
-      if (std::strcmp(e, "0") == 0 && fits) t.wide = 0;
+      if (std::strcmp(e, "1") == 0) t.hess = kHessGlobal;
+      if (std::strcmp(e, "0") == 0 && fits) t.hess = kHessSquare;
     }
-    int base = lds_solver_floats(m.nv, 0, t.rj, t.wide);
+    int base = lds_solver_floats(m.nv, 0, t.rj, t.hess);
     const int fwd = lds_forward(m, false);
     if (fwd > base) base = fwd;
     if (base + 8 * kLdsRowsMin <= cap) {
       const int per_cu = cap / (base + 8 * kLdsRowsMin);
-      const int rows = (cap / per_cu - lds_solver_floats(m.nv, 0, t.rj, t.wide)) / 8;
+      const int rows = (cap / per_cu - lds_solver_floats(m.nv, 0, t.rj, t.hess)) / 8;
       t.rmax = rows < kLdsRowsMin ? kLdsRowsMin : rows > kLdsRowsMax ? kLdsRowsMax : rows;
     }
   }
@@ -342,7 +347,7 @@ Tune tune_for(const mjhModel& m, bool reg) {
   // LDS solver with kLdsRowsMax rows when that fits one workgroup; 32-lane
   // models reach the tail only past the big-world launch's 256 rows, rarely
   // enough to leave it the global-memory solver and its small LDS
-  t.tail_rows = !reg && lds_solver_floats(m.nv, kLdsRowsMax, 0, t.wide != 0) <= (int)(lds_cap() / sizeof(float))
+  t.tail_rows = !reg && lds_solver_floats(m.nv, kLdsRowsMax, 0, t.hess) <= (int)(lds_cap() / sizeof(float))
                     ? kLdsRowsMax
                     : 0;
   t.resident = fwd_resident(m, reg ? kRegTeam : kTeam, (int)(lds_cap() / sizeof(float)));
@@ -352,12 +357,12 @@ Tune tune_for(const mjhModel& m) { return tune_for(m, reg_path(m)); }
 // the tail launch: the global-memory solver's LDS and the LDS solver's
 // with the tail's row capacity
 int lds_tail(const mjhModel& m, const Tune& t) {
-  const int a = lds_tail(m, t.wide != 0);
-  const int b = t.tail_rows > 0 ? lds_solver_floats(m.nv, t.tail_rows, 0, t.wide != 0) : 0;
+  const int a = lds_tail(m, t.hess != kHessSquare);
+  const int b = t.tail_rows > 0 ? lds_solver_floats(m.nv, t.tail_rows, 0, t.hess) : 0;
   return a > b ? a : b;
 }
 int lds_solve(const mjhModel& m, const Tune& t) {
-  const int a = lds_solver_floats(m.nv, t.rmax, t.rj, t.wide != 0), b = lds_linalg(m);
+  const int a = lds_solver_floats(m.nv, t.rmax, t.rj, t.hess), b = lds_linalg(m);
   return a > b ? a : b;
 }
 int lds_solve(const mjhModel& m) { return lds_solve(m, tune_for(m)); }

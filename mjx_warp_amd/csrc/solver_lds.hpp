@@ -22,12 +22,152 @@ namespace mjh {
 
 constexpr int kFlagDeferred = 1;
 
-// LDS floats per world: nv^2 (H; when wide H is in efc_h and this is the
-// blocked Cholesky's panel buffer) + 14 nv (vectors) + 8 rmax (rows) + rj nv
-// (staged Jacobian rows).  The mass
+// Where the Newton Hessian lives: kHessSquare, all of it in LDS; kHessGlobal,
+// in efc_h with the blocked Cholesky's panel buffer in LDS; kHessTri, its
+// lower triangle packed by rows in LDS, two rows per lane (nv <= kTriMax).
+enum { kHessSquare = 0, kHessGlobal = 1, kHessTri = 2 };
+constexpr int kTriMax = 128;
+
+// LDS floats per world: the Hessian (or its panel buffer) + 14 nv (vectors) +
+// 8 rmax (rows) + rj nv (staged Jacobian rows).  The mass
 // matrix is read from global memory, where it is read-only during the solve.
-__host__ __device__ inline int lds_solver_floats(int nv, int rmax, int rj, bool wide = false) {
-  return (wide ? chol_blocked_floats(nv) : nv * nv) + 14 * nv + 8 * rmax + rj * nv;
+__host__ __device__ inline int lds_solver_floats(int nv, int rmax, int rj, int hess = kHessSquare) {
+  const int h = hess == kHessGlobal ? chol_blocked_floats(nv) : hess == kHessTri ? nv * (nv + 1) / 2 : nv * nv;
+  return h + 14 * nv + 8 * rmax + rj * nv;
+}
+
+MJH_DEV int tri_row(int i) { return i * (i + 1) / 2; }
+MJH_DEV float lane_value(float v, int k) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+}
+
+// Cholesky factor of the packed lower triangle A (n <= kTriMax) by one
+// 64-lane team, in place.  Lane l owns rows l and l + 64, and nobody else
+// touches them: a panel of kTriPanel columns is factored with the rows'
+// entries in registers, the diagonal rows' read by readlane, and the rows'
+// later entries then take the panel's products column by column, the column's
+// row of the panel read by readlane as well -- no barrier and no LDS word
+// shared between lanes (row starts are triangular numbers, distinct modulo
+// the banks).  Each entry gets the operations of chol_lds in its order, so
+// the factor is the same bit for bit.  Bound by the serial chain of square
+// root, reciprocal and broadcasts down the diagonal, where chol_lds passes
+// every column through LDS with three barriers (170 us at nv 81) and
+// chol_blocked goes to efc_h in global memory (205 us): 1024 worlds of three
+// attached humanoids step in 2.23 ms with it, 4.53 ms before.
+constexpr int kTriPanel = 16;
+// One panel from column p on: r0, r1 the lane's rows.  kHigh: the panel's
+// diagonal rows are the lanes' second rows (p >= 64), the first are done.
+// Columns past n work on zeros (and what comes of them), which nobody keeps.
+template <bool kHigh>
+MJH_DEV void chol_tri_panel(float* r0, float* r1, int n, int p, int lane) {
+  constexpr int B = kTriPanel;
+  const int i1 = lane + 64, q0 = kHigh ? p - 64 : p;  // the lane of the first diagonal row
+  const bool own0 = !kHigh && lane < n, own1 = i1 < n;
+  float x0[B], x1[B];
+#pragma unroll
+  for (int k = 0; k < B; k++) {
+    x0[k] = own0 && lane >= p + k ? r0[p + k] : 0.0f;
+    x1[k] = own1 && i1 >= p + k ? r1[p + k] : 0.0f;
+  }
+#pragma unroll
+  for (int k = 0; k < B; k++) {
+    const float dkk = sqrtf(lane_value(kHigh ? x1[k] : x0[k], q0 + k));
+    const float inv = 1.0f / dkk;
+    if (!kHigh) x0[k] = lane == q0 + k ? dkk : x0[k] * inv;
+    x1[k] = kHigh && lane == q0 + k ? dkk : x1[k] * inv;
+#pragma unroll
+    for (int j = k + 1; j < B; j++) {
+      const float l = lane_value(kHigh ? x1[k] : x0[k], q0 + j);
+      if (!kHigh) x0[j] = fmaf(-x0[k], l, x0[j]);
+      x1[j] = fmaf(-x1[k], l, x1[j]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < B; k++) {
+    if (own0 && lane >= p + k) r0[p + k] = x0[k];
+    if (own1 && i1 >= p + k) r1[p + k] = x1[k];
+  }
+  int c = p + B;
+  if (!kHigh) {
+    const int c64 = n < 64 ? n : 64;
+#pragma unroll 2
+    for (; c < c64; c++) {
+      const bool u0 = own0 && lane >= c;
+      float a0 = u0 ? r0[c] : 0.0f, a1 = own1 ? r1[c] : 0.0f;
+#pragma unroll
+      for (int k = 0; k < B; k++) {
+        const float l = lane_value(x0[k], c);
+        a0 = fmaf(-x0[k], l, a0);
+        a1 = fmaf(-x1[k], l, a1);
+      }
+      if (u0) r0[c] = a0;
+      if (own1) r1[c] = a1;
+    }
+  }
+#pragma unroll 2
+  for (; c < n; c++) {
+    const bool u1 = own1 && i1 >= c;
+    float a1 = u1 ? r1[c] : 0.0f;
+#pragma unroll
+    for (int k = 0; k < B; k++) a1 = fmaf(-x1[k], lane_value(x1[k], c - 64), a1);
+    if (u1) r1[c] = a1;
+  }
+}
+MJH_DEV void chol_tri(float* A, int n, int lane) {
+  static_assert(64 % kTriPanel == 0, "a panel's diagonal rows are one set of rows");
+  float* const r0 = A + tri_row(lane < n ? lane : 0);
+  float* const r1 = A + tri_row(lane + 64 < n ? lane + 64 : 0);
+#pragma unroll 1
+  for (int p = 0; p < n && p < 64; p += kTriPanel) chol_tri_panel<false>(r0, r1, n, p, lane);
+#pragma unroll 1
+  for (int p = 64; p < n; p += kTriPanel) chol_tri_panel<true>(r0, r1, n, p, lane);
+  wave_fence();
+}
+
+// x = inv(L L') x for the packed factor, x one entry per lane and set (lanes
+// l and l + 64); each entry gets the operations of cho_solve_wave in its
+// order.  The rows' words do not depend on the chain and are loaded ahead.
+MJH_DEV void cho_solve_tri(const float* A, int n, float* x0, float* x1, int lane) {
+  const int i1 = lane + 64;
+  const bool own0 = lane < n, own1 = i1 < n;
+  const float* const r0 = A + tri_row(own0 ? lane : 0);
+  const float* const r1 = A + tri_row(own1 ? i1 : 0);
+  const float l0 = own0 ? r0[lane] : 1.0f, l1 = own1 ? r1[i1] : 1.0f;
+  float y0 = own0 ? *x0 : 0.0f, y1 = own1 ? *x1 : 0.0f;
+  const int c64 = n < 64 ? n : 64;
+#pragma unroll 8
+  for (int k = 0; k < c64; k++) {
+    const float a0 = lane > k && own0 ? r0[k] : 0.0f, a1 = own1 ? r1[k] : 0.0f;
+    const float yk = lane_value(y0 / l0, k);
+    if (lane == k) y0 = yk;
+    else if (lane > k) y0 = fmaf(-a0, yk, y0);
+    y1 = fmaf(-a1, yk, y1);
+  }
+#pragma unroll 8
+  for (int k = 64; k < n; k++) {
+    const float a1 = i1 > k && own1 ? r1[k] : 0.0f;
+    const float yk = lane_value(y1 / l1, k - 64);
+    if (i1 == k) y1 = yk;
+    else if (i1 > k) y1 = fmaf(-a1, yk, y1);
+  }
+#pragma unroll 8
+  for (int k = n - 1; k >= 64; k--) {
+    const float* const row = A + tri_row(k);
+    const float a0 = row[lane], a1 = i1 < k ? row[i1] : 0.0f;
+    const float xk = lane_value(y1 / l1, k - 64);
+    if (i1 == k) y1 = xk;
+    else if (i1 < k) y1 = fmaf(-a1, xk, y1);
+    y0 = fmaf(-a0, xk, y0);
+  }
+#pragma unroll 8
+  for (int k = c64 - 1; k >= 0; k--) {
+    const float a0 = lane < k ? A[tri_row(k) + lane] : 0.0f;
+    const float xk = lane_value(y0 / l0, k);
+    if (lane == k) y0 = xk;
+    else if (lane < k) y0 = fmaf(-a0, xk, y0);
+  }
+  *x0 = y0;
+  *x1 = y1;
 }
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -40,37 +180,56 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 // as the A operand, J[r][tj*32 + c] as the B operand; result entry v of lane
 // l is tile row 8 (v / 4) + 4 (l / 32) + v % 4, tile column l % 32.  Every
 // lane of the wavefront must call it (the matrix instruction uses all 64).
+// tri: H packed by rows (tri_row) instead of row stride nv.  A row of tiles
+// is accumulated together: its Jacobian entries are loaded once.
 MJH_DEV void hessian_mfma(const float* M, const float* J, const float* D, const float* act, int nr, int nv,
-                          float* H, int lane) {
+                          float* H, bool tri, int lane) {
   const int c = lane & 31, half = lane >> 5;
   const int nt = (nv + 31) >> 5;
   for (int ti = 0; ti < nt; ti++)
-    for (int tj = 0; tj <= ti; tj++) {
-      floatx16 acc = {};
-      const int ci = ti * 32 + c, cj = tj * 32 + c;
+    // four tiles at a time (nv <= 128: the whole row of tiles)
+    for (int t0 = 0; t0 <= ti; t0 += 4) {
+      floatx16 acc[4] = {};
+      const int ci = ti * 32 + c;
       // the operands of eight row pairs are loaded before their matrix
       // instructions, so that their loads are in flight together
       for (int k0 = 0; k0 < nr; k0 += 16) {
-        float a[8], b[8];
+        float a[8], b[4][8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
           const int r = k0 + 2 * u + half;
-          a[u] = 0.0f;
-          b[u] = 0.0f;
-          if (r < nr) {
-            const float dr = D[r] * act[r];
-            if (ci < nv) a[u] = dr * J[r * nv + ci];
-            if (cj < nv) b[u] = J[r * nv + cj];
+          const float dr = r < nr ? D[r] * act[r] : 0.0f;
+          a[u] = r < nr && ci < nv ? dr * J[r * nv + ci] : 0.0f;
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const int cj = (t0 + j) * 32 + c;
+            b[j][u] = t0 + j <= ti && r < nr && cj < nv ? J[r * nv + cj] : 0.0f;
           }
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u], b[u], acc, 0, 0, 0);
+        for (int j = 0; j < 4; j++)
+          if (t0 + j <= ti) {
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+              acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u], b[j][u], acc[j], 0, 0, 0);
+          }
       }
 #pragma unroll
-      for (int v = 0; v < 16; v++) {
-        const int i = ti * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
-        if (i < nv && cj < nv && cj <= i) H[i * nv + cj] = M[i * nv + cj] + acc[v];
-      }
+      for (int j = 0; j < 4; j++)
+        if (t0 + j <= ti) {
+          const int cj = (t0 + j) * 32 + c;
+          float mm[16];
+#pragma unroll
+          for (int v = 0; v < 16; v++) {
+            const int i = ti * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
+            mm[v] = i < nv && cj <= i ? M[i * nv + cj] : 0.0f;
+          }
+#pragma unroll
+          for (int v = 0; v < 16; v++) {
+            const int i = ti * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
+            if (i < nv && cj <= i) H[(tri ? tri_row(i) : i * nv) + cj] = mm[v] + acc[j][v];
+          }
+        }
     }
 }
 
@@ -84,7 +243,8 @@ struct LdsSolver {
   float *H, *qacc, *Ma, *grad, *Mgrad, *search, *mv, *qs, *qas, *qc, *pg, *pmg, *x;
   float *Jaref, *jv, *D, *q0, *q1, *q2, *force, *act;
   const float* J;  // row-major [nr, nv], LDS or global
-  float* pbuf = nullptr;  // wide: chol_blocked's panel buffer
+  float* pbuf = nullptr;  // kHessGlobal: chol_blocked's panel buffer
+  bool tri = false;       // kHessTri
   // Newton: the factor in H is current.  H = M + J' D(active) J depends on
   // the iterate only through the active set, so while no row changes
   // activity the previous factor is the one a rebuild would produce, bit
@@ -94,7 +254,30 @@ struct LdsSolver {
   bool fact_valid = false;
   unsigned act_bits = 0;
 
+  // blocks of M times vec; M is symmetric, so a lane reads its row as a
+  // column: coalesced, and every block at once
+  int mbeg[2], mend[2];  // the tree blocks of dofs t.lane and t.lane + TEAM
+  MJH_DEV void find_blocks() {
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const int i = t.lane + k * TEAM;
+      mbeg[k] = mend[k] = 0;
+      if (i < nv) tree_block(m, i, &mbeg[k], &mend[k]);
+    }
+  }
   MJH_DEV void mulM(float* res, const float* vec) const {
+    if (nv <= 2 * TEAM) {
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        const int i = t.lane + k * TEAM;
+        if (i >= nv) break;
+        float s = 0.0f;
+#pragma unroll 9
+        for (int c = mbeg[k]; c < mend[k]; c++) s += M[(size_t)c * nv + i] * vec[c];
+        res[i] = s;
+      }
+      return;
+    }
     for_each_tree_block(m, [&](int dof, int n) {
       for (int r = t.lane; r < n; r += TEAM) {
         float s = 0.0f;
@@ -124,6 +307,7 @@ struct LdsSolver {
     float g = 0.0f;
     for (int i = t.lane; i < nv; i += TEAM) {
       float s = 0.0f;
+#pragma unroll 8
       for (int r = 0; r < nr; r++) s += J[r * nv + i] * force[r];
       qc[i] = s;
       g += 0.5f * (Ma[i] - qs[i]) * (qacc[i] - qas[i]);
@@ -157,14 +341,20 @@ struct LdsSolver {
       act_bits = bits;
       fact_valid = true;
     }
-    if (m.opt.solver == mjhSOL_NEWTON && !refactor) {
+    if (TEAM == 64 && m.opt.solver == mjhSOL_NEWTON && refactor) {
+      hessian_mfma(M, J, D, act, nr, nv, H, tri, t.lane);
       sync();
-      cho_solve_lds(H, nv, nv, x, t);
-    } else if (m.opt.solver == mjhSOL_NEWTON && TEAM == 64) {
-      hessian_mfma(M, J, D, act, nr, nv, H, t.lane);
-      sync();
-      if (pbuf) chol_blocked(H, nv, nv, pbuf, m, t);
+      if (tri) chol_tri(H, nv, t.lane);
+      else if (pbuf) chol_blocked(H, nv, nv, pbuf, m, t);
       else chol_lds(H, nv, nv, m, t);
+    }
+    if (TEAM == 64 && tri) {
+      float x0 = t.lane < nv ? x[t.lane] : 0.0f, x1 = t.lane + 64 < nv ? x[t.lane + 64] : 0.0f;
+      cho_solve_tri(H, nv, &x0, &x1, t.lane);
+      if (t.lane < nv) x[t.lane] = x0;
+      if (t.lane + 64 < nv) x[t.lane + 64] = x1;
+    } else if (m.opt.solver == mjhSOL_NEWTON && (!refactor || TEAM == 64)) {
+      sync();
       cho_solve_lds(H, nv, nv, x, t);
     } else if (m.opt.solver == mjhSOL_NEWTON) {
       const int ntri = nv * (nv + 1) / 2;
@@ -307,6 +497,7 @@ struct LdsSolver {
     for (int r = t.lane; r < nr; r += TEAM) {
       float s = 0.0f;
       const float* Jr = J + r * nv;
+#pragma unroll 9
       for (int i = 0; i < nv; i++) s += Jr[i] * search[i];
       jv[r] = s;
       const float jar = Jaref[r], dd = D[r];
@@ -354,7 +545,7 @@ struct LdsSolver {
 // Returns false (and leaves the world untouched) when the world's rows do
 // not fit the LDS row capacity.
 template <int TEAM>
-MJH_DEV bool solve_lds(const mjhModel& m, const mjhData& d, float* lds, int rmax, int rj, bool wide,
+MJH_DEV bool solve_lds(const mjhModel& m, const mjhData& d, float* lds, int rmax, int rj, int hess,
                        const Team<TEAM>& t) {
   if (!t.valid) return true;
   const int w = t.world, nv = m.nv;
@@ -363,15 +554,18 @@ MJH_DEV bool solve_lds(const mjhModel& m, const mjhData& d, float* lds, int rmax
   LdsSolver<TEAM> s{m, d, t, w, nv, radr, nr};
   float* p = lds;
   s.M = d.qMd + (size_t)w * nv * nv;
-  // wide: H in the world's efc_h (CG: its tree-block factor in qLDd)
+  const bool wide = hess == kHessGlobal;
+  // kHessGlobal: H in the world's efc_h (CG: its tree-block factor in qLDd)
   if (wide) {
     s.H = m.opt.solver == mjhSOL_CG ? d.qLDd + (size_t)w * nv * nv : d.efc_h + (size_t)w * nv * nv;
     s.pbuf = p;
     p += chol_blocked_floats(nv);
   } else {
+    s.tri = hess == kHessTri;
     s.H = p;
-    p += nv * nv;
+    p += s.tri ? nv * (nv + 1) / 2 : nv * nv;
   }
+  if (nv <= 2 * TEAM) s.find_blocks();
   s.qacc = p; p += nv;
   s.Ma = p; p += nv;
   s.grad = p; p += nv;
@@ -418,6 +612,7 @@ MJH_DEV bool solve_lds(const mjhModel& m, const mjhData& d, float* lds, int rmax
     const float* Jr = s.J + r * nv;
     const float arn = d.efc_aref[radr + r] / (float)nv;
     float a = 0.0f;
+#pragma unroll 9
     for (int i = 0; i < nv; i++) a += Jr[i] * s.qacc[i] - arn;
     s.Jaref[r] = a;
   }

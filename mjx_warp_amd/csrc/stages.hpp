@@ -25,15 +25,15 @@ namespace mjh {
 constexpr int kTeam = 64;
 
 // launch-time tuning of the solvers: the LDS solver's row capacity and
-// staged J rows; wide: the Newton Hessians of the 64-lane solvers live in
-// efc_h (global) instead of LDS, for models whose nv^2 does not fit;
+// staged J rows; hess: where the LDS solver's Newton Hessian lives (kHess...;
+// the global-memory solver's is in LDS for kHessSquare, else in efc_h);
 // tail_rows: the row capacity of the LDS solver in the tail launch (0: the
 // tail has only the global-memory solver); resident: the fused forward
 // launch keeps the world's state in LDS (fwd_resident)
 struct Tune {
   int rmax;
   int rj;
-  int wide;
+  int hess;
   int tail_rows;
   int resident;
 };
@@ -75,7 +75,7 @@ STAGE(StQaccSmooth, if (t.valid) for (int i = t.lane; i < m.nv; i += T) d.qacc[t
 template <int T>
 MJH_DEV bool solve_team(const mjhModel& m, const mjhData& d, float* l, const Team<T>& t, const Tune& tune) {
   if constexpr (T == kRegTeam) return solve_reg<2, false>(m, d, l, tune.rj, t);
-  else return solve_lds(m, d, l, tune.rmax, tune.rj, tune.wide != 0, t);
+  else return solve_lds(m, d, l, tune.rmax, tune.rj, tune.hess, t);
 }
 // Worlds the 32-lane solve launches leave to the big-world launch.
 MJH_DEV bool big_world(const mjhData& d, int w) { return d.njmax != 0 && big_rows(d.world_efc[2 * w + 1]); }
@@ -116,8 +116,8 @@ struct StTail {
     if (!t.valid || !(d.world_flags[t.world] & kFlagDeferred)) return;
     // the LDS solver with the tail's row capacity, else the global one
     bool solved = false;
-    if constexpr (T == kTeam) solved = tune.tail_rows > 0 && solve_lds(m, d, l, tune.tail_rows, 0, tune.wide != 0, t);
-    if (!solved) solve(m, d, l, t, tune.wide != 0);
+    if constexpr (T == kTeam) solved = tune.tail_rows > 0 && solve_lds(m, d, l, tune.tail_rows, 0, tune.hess, t);
+    if (!solved) solve(m, d, l, t, tune.hess != kHessSquare);
     sync();
     if (integrate) {
       if (m.opt.integrator == mjhINT_EULER) euler(m, d, l, t);
@@ -291,8 +291,16 @@ MJH_DEV const GroupDesc& group_of(const GroupDesc* __restrict__ g, int ngroups, 
   return g[lo];
 }
 
+// Wavefronts per SIMD that a stage's registers have to allow: two for the
+// 64-lane solver, whose unrolled panels and tiles otherwise take the 512
+// registers of one.
+template <class S>
+inline constexpr int kMinWaves = 1;
+template <>
+inline constexpr int kMinWaves<StSolveStep> = 2;
+
 template <int TEAM, class S, int TI>
-__global__ void __launch_bounds__(64) k_stage_groups(const GroupDesc* __restrict__ g, int ngroups, int lds_per_world) {
+__global__ void __launch_bounds__(64, kMinWaves<S>) k_stage_groups(const GroupDesc* __restrict__ g, int ngroups, int lds_per_world) {
   extern __shared__ float smem[];
   const int b = blockIdx.x;
   const GroupDesc& G = group_of(g, ngroups, b);
@@ -317,7 +325,7 @@ __global__ void __launch_bounds__(64) k_stage_groups(const GroupDesc* __restrict
 constexpr int kQueueLanes = 8;
 constexpr int kQueueStride = 64;
 template <int TEAM, class S, int TI>
-__global__ void __launch_bounds__(64) k_stage_queue(const GroupDesc* __restrict__ g, int ngroups, int lds_per_world,
+__global__ void __launch_bounds__(64, kMinWaves<S>) k_stage_queue(const GroupDesc* __restrict__ g, int ngroups, int lds_per_world,
                                                     int* queue, int nblocks) {
   extern __shared__ float smem[];
   const int c = blockIdx.x % kQueueLanes;
