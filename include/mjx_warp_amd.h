@@ -378,9 +378,11 @@ typedef struct mjhOption {
  * Size aliases: nworld2 = 2*nworld, nworld1 = nworld+1,
  * nworld_ngeom = nworld*ngeom. */
 
+#ifndef MJH_X_FIELD_R /* the library's own sources wrap the same pointers */
 #define MJH_X_FIELD_R(name) float* name;
 #define MJH_X_FIELD_I(name) int32_t* name;
 #define MJH_X_FIELD_B(name) uint8_t* name;
+#endif
 #define MJH_X_FIELD(kind, name, dims) MJH_X_FIELD_##kind(name)
 #define MJH_X_SIZE(name) int32_t name;
 

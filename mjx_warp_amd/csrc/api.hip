@@ -796,7 +796,7 @@ int solve_reg_desc(const mjhModel& m, const mjhData& d, hipStream_t s) {
   const int l_solve = lds_solve_reg(m), l_big = lds_tail_reg(m);
   if ((size_t)max_of(2 * l_solve, 2 * l_big) * sizeof(float) > lds_cap())
     return fail(MJH_ERR_CAPACITY, "solve: model too large for the dense LDS kernels (nv = " + std::to_string(m.nv) + ")");
-  GroupDesc* dev = reinterpret_cast<GroupDesc*>(d.step_desc);
+  GroupDesc* dev = reinterpret_cast<GroupDesc*>((int32_t*)d.step_desc);
   hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(256), 0, s, single_desc(m, d), dev, 0);
   TRY(check_launch("solve: description"));
   GroupTable t32;
@@ -815,7 +815,7 @@ int do_step_fused_desc(const mjhModel& m, const mjhData& d, hipStream_t s) {
   g.first_block = 0;
   g.tune[0] = tune_for(m);
   g.tune[1] = reg_path(m) ? tune_tail_reg(m) : g.tune[0];
-  GroupDesc* dev = reinterpret_cast<GroupDesc*>(d.step_desc);
+  GroupDesc* dev = reinterpret_cast<GroupDesc*>((int32_t*)d.step_desc);
   const bool reg = reg_path(m);
   const int l_fwd = lds_forward_reg(m), l_solve = lds_solve_reg(m), l_big = lds_tail_reg(m), l_step = lds_step(m),
             l_tail = lds_tail(m, g.tune[0]), l_fwd64 = max_of(lds_forward(m, false), lds_linalg(m)),
@@ -1307,7 +1307,7 @@ size_t tape_plan(const mjhModel& m, const mjhData& d, char* slot, mjhData* out, 
     off = (off + 255) & ~(size_t)255;
     if (segs && k < kTapeSegsMax) segs->s[k] = TapeSeg{(const char*)src, off, bytes, count, row};
     k++;
-    field = reinterpret_cast<std::remove_reference_t<decltype(field)>>(slot + off);
+    field.set(slot + off);
     off += bytes;
   };
   const size_t W = d.nworld, nv = m.nv, nb = m.nbody, nu = m.nu, ng = m.ngeom, F = 4;

@@ -13,9 +13,30 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "../../include/mjx_warp_amd.h"
-
 #define MJH_DEV __device__ __forceinline__
+
+namespace mjh {
+// A field of mjhModel / mjhData as the kernels see it: a pointer that the
+// compiler knows to be to global memory.  The descriptions are read from
+// memory, so a plain pointer taken from them could be to anything: its
+// accesses compile to flat instructions, which count as LDS accesses too, and
+// every wait for an LDS word then waits for all loads and stores in flight.
+template <class T>
+struct Glob {
+#ifdef __HIP_DEVICE_COMPILE__
+  __attribute__((address_space(1))) T* p;
+#else
+  T* p;
+#endif
+  __host__ __device__ operator T*() const { return (T*)p; }
+  __host__ __device__ void set(void* q) { p = (decltype(p))q; }
+};
+}  // namespace mjh
+#define MJH_X_FIELD_R(name) mjh::Glob<float> name;
+#define MJH_X_FIELD_I(name) mjh::Glob<int32_t> name;
+#define MJH_X_FIELD_B(name) mjh::Glob<uint8_t> name;
+#include "../../include/mjx_warp_amd.h"
+static_assert(sizeof(mjh::Glob<float>) == sizeof(float*), "the fields are the header's pointers");
 
 // Per-world base pointer into a world-major Data array.
 #define WPTR(arr, w, stride) ((arr) + (size_t)(w) * (size_t)(stride))

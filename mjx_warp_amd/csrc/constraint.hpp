@@ -71,7 +71,7 @@ MJH_DEV bool big_rows(int nr) { return nr > kBigRowsMin && nr <= kBigRowsMax; }
 constexpr int kBigMapWord = MJH_STEP_DESC_WORDS / 2;
 constexpr int kBigMapWorlds = 32 * (MJH_STEP_DESC_WORDS - kBigMapWord);
 MJH_DEV unsigned* big_map(const mjhData& d) {
-  return d.step_desc && d.nworld <= kBigMapWorlds ? reinterpret_cast<unsigned*>(d.step_desc) + kBigMapWord : nullptr;
+  return d.step_desc && d.nworld <= kBigMapWorlds ? reinterpret_cast<unsigned*>((int32_t*)d.step_desc) + kBigMapWord : nullptr;
 }
 MJH_DEV void mark_big_world(const mjhData& d, int w, int nr) {
   unsigned* map = big_map(d);
