@@ -575,8 +575,22 @@ int reset(const mjhData& d, hipStream_t s, int which) {
 
 
 
+// A stage of sweep-and-prune collision, kSapWaves wavefronts a world.
+template <class S>
+int launch_waves(const mjhModel& m, const mjhData& d, hipStream_t s, int words, const char* name) {
+  if (d.nworld <= 0) return MJH_OK;
+  const size_t bytes = words * sizeof(float);
+  TRY(allow_lds(reinterpret_cast<const void*>(&k_stage_waves<S>), bytes, name));
+  hipLaunchKernelGGL((k_stage_waves<S>), dim3(d.nworld), dim3(kTeam * kSapWaves), bytes, s, m, d);
+  return check_launch(name);
+}
+
 int do_collision(const mjhModel& m, const mjhData& d, hipStream_t s) {
-  TRY(launch<StBroadphase>(m, d, s, lds_broadphase(m), "broadphase"));
+  if (m.ngeom > 100) {
+    TRY(launch_waves<StSapWaves>(m, d, s, lds_sap(m), "broadphase"));
+    return launch_waves<StNarrowWaves>(m, d, s, kNarrowWords, "narrowphase");
+  }
+  TRY(launch<StNxn>(m, d, s, lds_broadphase(m), "broadphase"));
   return launch<StNarrowphase>(m, d, s, 0, "narrowphase");
 }
 
@@ -1074,9 +1088,12 @@ int mjh_nxn_broadphase(const mjhModel* m, const mjhData* d, mjhStream stream) {
 }
 int mjh_sap_broadphase(const mjhModel* m, const mjhData* d, mjhStream stream) {
   TRY(reset(*d, (hipStream_t)stream, 1));
+  if (m->ngeom > 100) return launch_waves<StSapWaves>(*m, *d, (hipStream_t)stream, lds_sap(*m), "sap_broadphase");
   return launch<StSap>(*m, *d, (hipStream_t)stream, lds_sap(*m), "sap_broadphase");
 }
 int mjh_primitive_narrowphase(const mjhModel* m, const mjhData* d, mjhStream stream) {
+  if (m->ngeom > 100)
+    return launch_waves<StNarrowWaves>(*m, *d, (hipStream_t)stream, kNarrowWords, "primitive_narrowphase");
   return launch<StNarrowphase>(*m, *d, (hipStream_t)stream, 0, "primitive_narrowphase");
 }
 int mjh_collision(const mjhModel* m, const mjhData* d, mjhStream stream) {

@@ -59,7 +59,6 @@ STAGE(StComVel, com_vel(m, d, l, t))
 STAGE(StPassive, passive(m, d, t))
 STAGE(StNxn, nxn_broadphase(m, d, l, t))
 STAGE(StSap, sap_broadphase(m, d, l, t))
-STAGE(StBroadphase, if (m.ngeom <= 100) nxn_broadphase(m, d, l, t); else sap_broadphase(m, d, l, t))
 STAGE(StNarrowphase, narrowphase(m, d, t))
 STAGE(StMakeConstraint, make_constraint(m, d, l, t))
 STAGE(StFwdVelocity, fwd_velocity(m, d, l, t))
@@ -254,6 +253,26 @@ __global__ void __launch_bounds__(64) k_stage(mjhModel m, mjhData d, int lds_per
   S()(m, d, smem + t.slot * lds_per_world, t, tune);
 }
 
+// A stage of which kSapWaves wavefronts share one world (64-lane teams).
+struct StSapWaves {
+  MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<kTeam>& t) const {
+    sap_broadphase<kTeam, kSapWaves>(m, d, l, t);
+  }
+};
+struct StNarrowWaves {
+  MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<kTeam>& t) const {
+    narrowphase<kTeam, kSapWaves>(m, d, t, reinterpret_cast<int*>(l));
+  }
+};
+template <class S>
+__global__ void __launch_bounds__(kTeam * kSapWaves) k_stage_waves(mjhModel m, mjhData d) {
+  extern __shared__ float smem[];
+  Team<kTeam> t(d.nworld);
+  t.world = blockIdx.x;
+  t.valid = true;
+  S()(m, d, smem, t);
+}
+
 // counter reset without memset nodes (capture-safe), by one workgroup:
 // which bit 0: ncollision + ncon, bit 1: nefc and the big-world map
 MJH_DEV void reset_counters(const mjhData& d, int which) {
@@ -363,7 +382,7 @@ using StTailStep = StTail<true>;
   X(32, StFwdAcceleration) X(64, StFwdAcceleration) X(32, StQaccSmooth) X(64, StQaccSmooth)
 // broadphase, narrowphase, constraint rows
 #define MJH_KERNELS_COLLISION(X, G)                                                              \
-  X(32, StNxn) X(64, StNxn) X(32, StSap) X(64, StSap) X(32, StBroadphase) X(64, StBroadphase)     \
+  X(32, StNxn) X(64, StNxn) X(32, StSap) X(64, StSap)                       \
   X(32, StNarrowphase) X(64, StNarrowphase) X(32, StMakeConstraint) X(64, StMakeConstraint)
 // integrators, the LDS solver and the global-memory tail
 #define MJH_KERNELS_INTEGRATE(X, G) \
