@@ -40,11 +40,38 @@ MJH_DEV void wave_fence() {
   asm volatile("" ::: "memory");
 }
 
-// Value of v in lane k of this lane's team (k wave-uniform).
-MJH_DEV float bcast32(float v, int k) {
-  const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
-  const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k + 32));
-  return (threadIdx.x & 32) ? hi : lo;
+// `yes` in the lanes of a constant mask (over the 32 lanes of a team), `no` in
+// the others.  The mask is two scalar moves at its use, where a comparison
+// with the lane number is a vector instruction for each column, and masks that
+// the compiler knows of leave a loop for scalar registers that it then spills.
+template <unsigned MASK>
+MJH_DEV float pick(float yes, float no) {
+  float r;
+  asm("s_mov_b32 vcc_lo, %3\n\ts_mov_b32 vcc_hi, vcc_lo\n\tv_cndmask_b32_e32 %0, %1, %2, vcc"
+      : "=v"(r) : "v"(no), "v"(yes), "i"(MASK) : "vcc");
+  return r;
+}
+// lane k, and the lanes past k
+constexpr unsigned lane_mask(int k) { return 1u << k; }
+constexpr unsigned past_mask(int k) { return k < 31 ? ~0u << (k + 1) : 0u; }
+// y - z[k] h in one 16-lane row of each team (HIGH: the upper), z[k] from lane
+// k of that row.  The wait is for a z written just before.
+template <int K, bool HIGH>
+MJH_DEV void sub_row(float* y, float z, float h) {
+  if constexpr (HIGH)
+    asm("s_nop 1\n\tv_fmac_f32_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xa bank_mask:0xf"
+        : "+v"(*y) : "v"(z), "v"(h), "i"(K));
+  else
+    asm("s_nop 1\n\tv_fmac_f32_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0x5 bank_mask:0xf"
+        : "+v"(*y) : "v"(z), "v"(h), "i"(K));
+}
+// Calls f(std::integral_constant<int, k>) for k = B .. E - 1.
+template <int B, int E, class F>
+MJH_DEV void unrolled(F f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    unrolled<B + 1, E>(f);
+  }
 }
 
 // p, opaque to the optimiser: address arithmetic on it is redone at each use
@@ -154,7 +181,7 @@ struct RegChol {
   }
 
   // The lower factor's row `lane` from global memory, restricted to the
-  // lane's block (from column beg up to the diagonal), by way of the staging
+  // lane's block (from column beg to before the diagonal), by way of the staging
   // buffer `rows` (NVC rows): a row per lane read in place touches a cache
   // line per lane with every load.
   MJH_DEV void load_lower(const float* L, int nv, int beg, float* rows) {
@@ -175,7 +202,7 @@ struct RegChol {
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const int j = 4 * q + u;
-        h[j] = (dof && j >= beg && j <= ln) ? e[u] : (j == ln ? 1.0f : 0.0f);
+        h[j] = (dof && j >= beg && j < ln) ? e[u] : 0.0f;
       }
     }
     rdiag = dof ? 1.0f / rows[ln * JS + ln] : 1.0f;
@@ -185,21 +212,19 @@ struct RegChol {
   MJH_DEV void divide_diag(const float* rows, int nv) { rdiag = lane < nv ? 1.0f / rows[lane * JS + lane] : 1.0f; }
 
   // Cholesky H = L L' of the lane-owned rows (right-looking, one column
-  // broadcast through LDS per step).  Lane i keeps L[i][0..i] in h[0..i]
-  // and 1 / L[i][i] in rdiag.
-  // kDiag unset: the diagonal of L is not kept, for a factor that solve()
-  // alone reads.  rsq: 1 / L[i][i] from one reciprocal square root, which
+  // broadcast through LDS per step).  Lane i keeps L[i][0..i-1] in h[0..i-1],
+  // zeros from there on and 1 / L[i][i] in rdiag: what solve() reads.
+  // kDiag: the diagonal of L is in h[i] too, to be stored (drop_diag() then
+  // makes it a factor for solve()).  rsq: 1 / L[i][i] from one reciprocal square root, which
   // differs from square root and reciprocal in the last bit (callers keep the
   // form they have, so that their results stay as they are).
   template <bool kDiag = true>
   MJH_DEV void factor(bool rsq = false) {
-    // this call's own lane number: comparisons with it are made where they
-    // are used instead of being kept in (and spilled from) scalar registers
-    const int ln = opaque(lane);
-#pragma unroll
-    for (int k = 0; k < NVC; k++) {
-      wave_fence();
-      cbuf[ln] = h[k];
+    const int ln = lane;
+    wave_fence();
+    cbuf[ln] = h[0];
+    unrolled<0, NVC>([&](auto col) {
+      constexpr int k = col;
       wave_fence();
       float c[NVC];
 #pragma unroll
@@ -212,38 +237,116 @@ struct RegChol {
       }
       const float dkk = c[k];
       float lkk = __builtin_amdgcn_sqrtf(dkk);
-      asm volatile("" : "+v"(lkk));  // else the compiler may make a rsq of the two
+      asm("" : "+v"(lkk));  // else the compiler may make a rsq of the two
       const float inv = rsq ? __builtin_amdgcn_rsqf(dkk) : __builtin_amdgcn_rcpf(lkk);
       // L[i][k] L[j][k] = H[i][k] H[j][k] / dkk
-      const float g = ln > k ? h[k] * (inv * inv) : 0.0f;
+      const float hk = pick<past_mask(k)>(h[k], 0.0f);
+      const float g = hk * (inv * inv);
+      // the next column first, and on its way to the other lanes while the rest
+      // is worked
+      if constexpr (k + 1 < NVC) {
+        h[k + 1] = fmaf(-g, c[k + 1], h[k + 1]);
+        wave_fence();
+        cbuf[ln] = h[k + 1];
+      }
 #pragma unroll
-      for (int j = k + 1; j < NVC; j++) h[j] = fmaf(-g, c[j], h[j]);
-      if (ln == k) rdiag = inv;
-      if (kDiag) h[k] = ln > k ? h[k] * inv : (ln == k ? lkk : h[k]);
-      else h[k] *= inv;  // solve() reads it in the lanes past k only
-    }
+      for (int j = k + 2; j < NVC; j++) h[j] = fmaf(-g, c[j], h[j]);
+      rdiag = pick<lane_mask(k)>(inv, rdiag);
+      h[k] = hk * inv;
+      if (kDiag) h[k] = pick<lane_mask(k)>(lkk, h[k]);
+    });
+  }
+  MJH_DEV void drop_diag() {
+    unrolled<0, NVC>([&](auto k) { h[k] = pick<lane_mask(k)>(0.0f, h[k]); });
   }
 
-  // x = inv(L L') b with L from factor() / load_lower(); b, x one entry per
-  // lane (padding lanes carry 0)
+  // x = inv(L L') b with L from factor() / load_lower() (h zero from the
+  // diagonal on); b, x one entry per lane (padding lanes carry 0).
+  // The two substitutions are a serial chain of NVC steps each, and where
+  // wavefronts are many their instructions are what the solver issues, so a
+  // step is kept inside the 16-lane row that owns it: its value comes by the
+  // row's own broadcast within the multiply-add, and what one row owes the
+  // other passes at once, when the row is done.  (A value for both rows at every
+  // step, masks compared with the lane number and five-level sums were 680
+  // vector instructions at 28 columns; these are 362.  8192 humanoids 908 to 880 us
+  // for two steps, 24576 lying ones 3773 to 3682.)
   MJH_DEV float solve(float b) const {
-    const int ln = opaque(lane);
+    constexpr int N0 = NVC < 16 ? NVC : 16;
     // forward: y = inv(L) b, column by column
     float y = b;
-#pragma unroll
-    for (int k = 0; k < NVC; k++) {
-      const float yk = bcast32(y * rdiag, k);
-      y = ln > k ? fmaf(-h[k], yk, y) : y;
+    unrolled<0, N0>([&](auto k) { sub_row<k, false>(&y, y * rdiag, h[k]); });
+    if constexpr (NVC > 16) {
+      const float z = __int_as_float(swap_rows(__float_as_int(y * rdiag)).even);
+      unrolled<0, 16>([&](auto k) { sub_row<k, true>(&y, z, h[k]); });
+      unrolled<16, NVC>([&](auto k) { sub_row<k - 16, true>(&y, y * rdiag, h[k]); });
     }
     y *= rdiag;
-    // backward: x = inv(L') y, x[k] = (y[k] - sum_{j>k} L[j][k] x[j]) / L[k][k]
+    asm("" : "+v"(y));  // rounded here, not within the differences below
+    // backward: x = inv(L') y, x[k] = (y[k] - sum_{j>k} L[j][k] x[j]) / L[k][k],
+    // the sums in the order of sum32.  The lanes j <= k have a zero L or a
+    // zero x, so the levels that would add only those are left out.
     float x = 0.0f;
-#pragma unroll
-    for (int k = NVC - 1; k >= 0; k--) {
-      const float s = sum32(ln > k ? h[k] * x : 0.0f);
-      if (ln == k) x = (y - s) * rdiag;
-    }
+    auto row_sum = [&](int k) {
+      float p = h[k] * x;
+      asm("" : "+v"(p));
+      p += dpp_f<0xB1>(p);
+      p += dpp_f<0x4E>(p);
+      if ((k & 15) < 12) p += dpp_f<0x141>(p);
+      if ((k & 15) < 8) p += dpp_f<0x140>(p);
+      return p;
+    };
+    unrolled<0, NVC - N0>([&](auto i) {
+      constexpr int k = NVC - 1 - i;
+      x = pick<lane_mask(k)>((y - row_sum(k)) * rdiag, x);
+    });
+    float upper = 0.0f;
+    if constexpr (NVC > 16) upper = __int_as_float(swap_rows(__float_as_int(upper_sums(x))).odd);
+    unrolled<0, N0>([&](auto i) {
+      constexpr int k = N0 - 1 - i;
+      float s = row_sum(k);
+      if (NVC > 16) s += upper;
+      x = pick<lane_mask(k)>((y - s) * rdiag, x);
+    });
     return x;
+  }
+
+  // In lane l the sum over l's row of L[j][l % 16] x[j], added as sum32 adds a
+  // row: of the 16 columns' sums each level hands the half that the partner
+  // lane keeps to it (15 adds for 16 sums of four levels).  Lane l keeps the
+  // column c = l % 16 through all levels: level 1 decides bit 0 ^ bit 2 of c,
+  // level 2 bit 1 ^ bit 2, level 3 bit 2 ^ bit 3 and level 4 bit 3, each of
+  // which differs between that level's partners and is the same between those
+  // of all later ones (l ^ 1, l ^ 2, l ^ 7, l ^ 15).
+  MJH_DEV float upper_sums(float x) const {
+    float a[16], b[8], c[4], e[2];
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+      a[k] = h[k] * x;
+      asm("" : "+v"(a[k]));
+    }
+    // lanes with bit 0 ^ bit 2, bit 1 ^ bit 2, bit 2 ^ bit 3, bit 3
+    constexpr unsigned m1 = 0x5a5a5a5au, m2 = 0x3c3c3c3cu, m3 = 0x0ff00ff0u, m4 = 0xff00ff00u;
+    // pairs of columns that differ in the level's bit and agree in the later
+    // levels': c and c ^ 1, then c ^ 2, c ^ 7 and c ^ 15
+#pragma unroll
+    for (int i = 0; i < 8; i++) {  // columns 2 i, 2 i + 1; the first has bit 0 ^ bit 2 = (i >> 1) & 1
+      const int f = (i >> 1) & 1;
+      const float lo = a[2 * i + f], hi = a[2 * i + 1 - f];
+      b[i] = pick<m1>(hi, lo) + dpp_f<0xB1>(pick<m1>(lo, hi));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {  // b[2 i], b[2 i + 1] are columns 4 i.. and 4 i + 2..
+      const int f = i & 1;
+      const float lo = b[2 * i + f], hi = b[2 * i + 1 - f];
+      c[i] = pick<m2>(hi, lo) + dpp_f<0x4E>(pick<m2>(lo, hi));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {  // c[2 i], c[2 i + 1] are columns 8 i.. and 8 i + 4..
+      const int f = i;
+      const float lo = c[2 * i + f], hi = c[2 * i + 1 - f];
+      e[i] = pick<m3>(hi, lo) + dpp_f<0x141>(pick<m3>(lo, hi));
+    }
+    return pick<m4>(e[1], e[0]) + dpp_f<0x140>(pick<m4>(e[0], e[1]));
   }
 
   // Writes the rows into the blocks [beg, end) of A (global, [nv, nv]) by

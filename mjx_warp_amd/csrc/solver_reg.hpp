@@ -211,7 +211,7 @@ struct RegSolver {
 #pragma unroll
         for (int j = 0; j < NVC; j++) ch.h[j] = fmaf(a, j < nv ? Jr[j < nv ? j : 0] : 0.0f, ch.h[j]);
       }
-      ch.factor();
+      ch.template factor<false>();
     }
     // (CG preconditions with the factor of M, in ch from the start)
     Mgrad = ch.solve(grad);
@@ -405,6 +405,7 @@ MJH_DEV bool solve_reg_nv(const mjhModel& m, const mjhData& d, float* lds, int r
     s.ch.factor();
     s.ch.store_rows(d.qLDd + o * nv, nv, beg, end, s.Jl, true);
     s.ch.divide_diag(s.Jl, nv);
+    s.ch.drop_diag();
     s.qas = s.ch.solve(s.qs);
     if (dof) d.qacc_smooth[o + lane] = s.qas;
     if (nr > 32 * RS) return false;
