@@ -273,7 +273,8 @@ int lds_linalg(const mjhModel& m) {
     const int r = lds_reg_matrix(reg_nvc(m.nv));
     if (r > a) a = r;
   }
-  return m.opt.is_sparse && m.nM > a ? m.nM : a;
+  const int sp = m.opt.is_sparse ? lds_sparse_words(m.nM, m.nv) : 0;
+  return sp > a ? sp : a;
 }
 // the global-memory solver of the tail launches: per-block linear algebra
 // and its Newton Hessian with right-hand side (nv^2 + nv), or when wide (H

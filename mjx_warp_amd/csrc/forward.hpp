@@ -416,6 +416,14 @@ MJH_DEV void euler(const mjhModel& m, const mjhData& d, float* lds, const Team<T
     float* qacc_int = WPTR(d.qacc_integration, w, nv);
     const float dt = m.opt.timestep;
     for_each_tree_block(m, [&](int dof, int n) {
+      if (n <= kTriMax) {
+        const float* const Mb = qM + dof * nv + dof;
+        tri_solve(lds, n, t.lane, false,
+                  [&](int r, int c) { return Mb[r * nv + c]; },
+                  [&](float& v, int i) { v += m.dof_damping[dof + i] * dt; },
+                  [&](int i) { return qs[dof + i] + qc[dof + i]; }, [&](int i, float v) { qacc_int[dof + i] = v; });
+        return;
+      }
       float* A = lds;
       float* x = lds + n * n;
       for (int p = t.lane; p < n * n; p += TEAM) {
@@ -484,6 +492,12 @@ MJH_DEV void implicit(const mjhModel& m, const mjhData& d, float* lds, const Tea
     const float* qfi = WPTR(d.qfrc_integration, w, nv);
     float* qacc_int = WPTR(d.qacc_integration, w, nv);
     for_each_tree_block(m, [&](int dof, int n) {
+      if (n <= kTriMax) {
+        const float* const Mb = qMi + dof * nv + dof;
+        tri_solve(lds, n, t.lane, false, [&](int r, int c) { return Mb[r * nv + c]; }, [](float&, int) {},
+                  [&](int i) { return qfi[dof + i]; }, [&](int i, float v) { qacc_int[dof + i] = v; });
+        return;
+      }
       float* A = lds;
       float* x = lds + n * n;
       for (int p = t.lane; p < n * n; p += TEAM) A[p] = qMi[(dof + p / n) * nv + dof + p % n];

@@ -246,30 +246,74 @@ MJH_DEV void dense_to_sparse(const mjhModel& m, const float* A, float* S, const 
   }
 }
 
+// LDS words of factor_sparse: the matrix and, up to kSparseTableMax words in
+// all, each entry's row start (dof_Madr of its column) and each row's (past
+// that they are read from the model: a matrix that fills the LDS by itself
+// stays as it was).
+constexpr int kSparseTableMax = 16384;
+__host__ __device__ inline bool sparse_table(int nM, int nv) { return 2 * nM + nv + 1 <= kSparseTableMax; }
+__host__ __device__ inline int lds_sparse_words(int nM, int nv) { return sparse_table(nM, nv) ? 2 * nM + nv + 1 : nM; }
+
 // smooth.py:317-350 _factor_i_sparse: the L'DL factor of the sparse matrix S
 // (global) into L (unit L below the diagonal, D on it) and Dinv = 1 / D,
-// leaves first as MuJoCo; worked in LDS (nM floats), lanes over the entries
-// of each updated row.  Every world runs the same loop (model-only bounds).
+// leaves first as MuJoCo; worked in LDS (lds_sparse_words).  Row k changes the
+// rows of its ancestors, each entry once, from entries of row k that keep
+// their values until all are done: four lanes take an ancestor, and all
+// ancestors of k go together.  What bounds it is the chain over the rows.  (One
+// ancestor at a time, its row looked up in global memory and two barriers
+// each, with the blocks' factors below: 146 us of factor_m a step for three
+// attached humanoids with the look-ups in LDS alone, 102 with packed blocks,
+// 86 with entries loaded ahead of their stores.)
 template <int TEAM>
 MJH_DEV void factor_sparse(const mjhModel& m, const float* S, float* L, float* Dinv, float* lds,
                            const Team<TEAM>& t) {
   const int nv = m.nv, nM = m.nM;
-  if (t.valid)
+  const bool table = sparse_table(nM, nv);
+  int* const ladr = reinterpret_cast<int*>(lds + nM);
+  int* const lrow = ladr + nM;
+  if (t.valid) {
     for (int k = t.lane; k < nM; k += TEAM) lds[k] = S[k];
-  sync();
-  for (int k = nv - 1; k >= 0; k--) {
-    const int ak = m.dof_Madr[k];
-    int p = 1;
-    for (int i = m.dof_parentid[k]; i >= 0; i = m.dof_parentid[i], p++) {
-      const float tmp = lds[ak + p] / lds[ak];
-      const int ai = m.dof_Madr[i];
-      const int len = m.dof_Madr[i + 1] - ai;  // i < k <= nv - 1
-      for (int q = t.lane; q < len; q += TEAM) lds[ai + q] -= lds[ak + p + q] * tmp;
-      sync();
-      if (t.lane == 0) lds[ak + p] = tmp;
-      sync();
+    if (table) {
+      for (int k = t.lane; k < nM; k += TEAM) ladr[k] = m.dof_Madr[m.qM_fullm_j[k]];
+      for (int k = t.lane; k <= nv; k += TEAM) lrow[k] = k < nv ? m.dof_Madr[k] : nM;
     }
   }
+  sync();
+  if (t.valid) {
+    const int l4 = t.lane % 4, p1 = 1 + t.lane / 4;
+    // the next row's start and its ancestors' are read a row ahead
+    auto row = [&](int k) { return k < 0 ? 0 : table ? lrow[k] : m.dof_Madr[k]; };
+    auto anc = [&](int e) { return table ? ladr[min(e, nM - 1)] : m.dof_Madr[m.qM_fullm_j[min(e, nM - 1)]]; };
+    int end = nM, ak = row(nv - 1), ai1 = anc(ak + p1);
+    for (int k = nv - 1; k >= 0; k--) {
+      const int n = end - ak, next = row(k - 1), ai1_next = anc(next + p1);
+      const float dk = lds[ak];
+      for (int p = p1; p < n; p += TEAM / 4) {
+        const int ai = p == p1 ? ai1 : anc(ak + p);
+        const float tmp = lds[ak + p] / dk;
+        for (int q0 = l4; q0 < n - p; q0 += 16) {
+          // four entries' loads before their stores
+          float a[4], b[4];
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            const int q = min(q0 + 4 * u, n - p - 1);
+            a[u] = lds[ak + p + q];
+            b[u] = lds[ai + q];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; u++)
+            if (q0 + 4 * u < n - p) lds[ai + q0 + 4 * u] = b[u] - a[u] * tmp;
+        }
+        wave_fence();
+        if (l4 == 0) lds[ak + p] = tmp;
+      }
+      wave_fence();
+      end = ak;
+      ak = next;
+      ai1 = ai1_next;
+    }
+  }
+  sync();
   if (t.valid) {
     for (int k = t.lane; k < nM; k += TEAM) L[k] = lds[k];
     for (int k = t.lane; k < nv; k += TEAM) Dinv[k] = 1.0f / lds[m.dof_Madr[k]];
@@ -532,8 +576,210 @@ MJH_DEV void cho_solve_lds(const float* L, int n, int ld, float* x, const Team<T
   }
 }
 
+// ---- packed lower triangles, one or two rows per lane of a 64-lane team ----
+constexpr int kTriMax = 128;
+MJH_DEV int tri_row(int i) { return i * (i + 1) / 2; }
+MJH_DEV float lane_value(float v, int k) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+}
+
+// Cholesky factor of the packed lower triangle A (n <= kTriMax) by one
+// 64-lane team, in place.  Lane l owns rows l and l + 64, and nobody else
+// touches them: a panel of kTriPanel columns is factored with the rows'
+// entries in registers, the diagonal rows' read by readlane, and the rows'
+// later entries then take the panel's products column by column, the column's
+// row of the panel read by readlane as well -- no barrier and no LDS word
+// shared between lanes (row starts are triangular numbers, distinct modulo
+// the banks).  Each entry gets the operations of chol_lds in its order, so
+// the factor is the same bit for bit.  Bound by the serial chain of square
+// root, reciprocal and broadcasts down the diagonal, where chol_lds passes
+// every column through LDS with three barriers (170 us at nv 81) and
+// chol_blocked goes to efc_h in global memory (205 us): 1024 worlds of three
+// attached humanoids step in 2.23 ms with it, 4.53 ms before.
+constexpr int kTriPanel = 16;
+// One panel from column p on: r0, r1 the lane's rows.  kHigh: the panel's
+// diagonal rows are the lanes' second rows (p >= 64), the first are done.
+// Columns past n work on zeros (and what comes of them), which nobody keeps.
+// kTwo unset: n <= 64, no second rows.
+template <bool kHigh, bool kTwo>
+MJH_DEV void chol_tri_panel(float* r0, float* r1, int n, int p, int lane) {
+  constexpr int B = kTriPanel;
+  const int i1 = lane + 64, q0 = kHigh ? p - 64 : p;  // the lane of the first diagonal row
+  const bool own0 = !kHigh && lane < n, own1 = kTwo && i1 < n;
+  float x0[B], x1[B];
+#pragma unroll
+  for (int k = 0; k < B; k++) {
+    x0[k] = own0 && lane >= p + k ? r0[p + k] : 0.0f;
+    x1[k] = own1 && i1 >= p + k ? r1[p + k] : 0.0f;
+  }
+#pragma unroll
+  for (int k = 0; k < B; k++) {
+    const float dkk = sqrtf(lane_value(kHigh ? x1[k] : x0[k], q0 + k));
+    const float inv = 1.0f / dkk;
+    if (!kHigh) x0[k] = lane == q0 + k ? dkk : x0[k] * inv;
+    if (kTwo) x1[k] = kHigh && lane == q0 + k ? dkk : x1[k] * inv;
+#pragma unroll
+    for (int j = k + 1; j < B; j++) {
+      const float l = lane_value(kHigh ? x1[k] : x0[k], q0 + j);
+      if (!kHigh) x0[j] = fmaf(-x0[k], l, x0[j]);
+      if (kTwo) x1[j] = fmaf(-x1[k], l, x1[j]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < B; k++) {
+    if (own0 && lane >= p + k) r0[p + k] = x0[k];
+    if (own1 && i1 >= p + k) r1[p + k] = x1[k];
+  }
+  int c = p + B;
+  if (!kHigh) {
+    const int c64 = n < 64 ? n : 64;
+#pragma unroll 2
+    for (; c < c64; c++) {
+      const bool u0 = own0 && lane >= c;
+      float a0 = u0 ? r0[c] : 0.0f, a1 = own1 ? r1[c] : 0.0f;
+#pragma unroll
+      for (int k = 0; k < B; k++) {
+        const float l = lane_value(x0[k], c);
+        a0 = fmaf(-x0[k], l, a0);
+        if (kTwo) a1 = fmaf(-x1[k], l, a1);
+      }
+      if (u0) r0[c] = a0;
+      if (own1) r1[c] = a1;
+    }
+  }
+#pragma unroll 2
+  for (; kTwo && c < n; c++) {
+    const bool u1 = own1 && i1 >= c;
+    float a1 = u1 ? r1[c] : 0.0f;
+#pragma unroll
+    for (int k = 0; k < B; k++) a1 = fmaf(-x1[k], lane_value(x1[k], c - 64), a1);
+    if (u1) r1[c] = a1;
+  }
+}
+MJH_DEV void chol_tri(float* A, int n, int lane) {
+  static_assert(64 % kTriPanel == 0, "a panel's diagonal rows are one set of rows");
+  float* const r0 = A + tri_row(lane < n ? lane : 0);
+  float* const r1 = A + tri_row(lane + 64 < n ? lane + 64 : 0);
+  if (n <= 64) {
+#pragma unroll 1
+    for (int p = 0; p < n; p += kTriPanel) chol_tri_panel<false, false>(r0, r1, n, p, lane);
+  } else {
+#pragma unroll 1
+    for (int p = 0; p < 64; p += kTriPanel) chol_tri_panel<false, true>(r0, r1, n, p, lane);
+#pragma unroll 1
+    for (int p = 64; p < n; p += kTriPanel) chol_tri_panel<true, true>(r0, r1, n, p, lane);
+  }
+  wave_fence();
+}
+
+// y / l given 1 / l: the quotient rounded from its residual, as a division ends,
+// without the scaling and the reciprocal that start one (a division is eleven
+// dependent instructions, and the solves below are a chain of 2 n of them).
+// div_fixup settles zeros, infinities and NaN.
+MJH_DEV float div_by(float y, float l, float inv) {
+  const float q = y * inv;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-l, q, y), inv, q), l, y);
+}
+
+// x = inv(L L') x for the packed factor, x one entry per lane and set (lanes
+// l and l + 64); each entry gets the operations of cho_solve_wave in its
+// order.  The rows' words do not depend on the chain and are loaded ahead.
+MJH_DEV void cho_solve_tri(const float* A, int n, float* x0, float* x1, int lane) {
+  const int i1 = lane + 64;
+  const bool own0 = lane < n, own1 = i1 < n;
+  const float* const r0 = A + tri_row(own0 ? lane : 0);
+  const float* const r1 = A + tri_row(own1 ? i1 : 0);
+  const float l0 = own0 ? r0[lane] : 1.0f, l1 = own1 ? r1[i1] : 1.0f;
+  const float v0 = 1.0f / l0, v1 = 1.0f / l1;
+  float y0 = own0 ? *x0 : 0.0f, y1 = own1 ? *x1 : 0.0f;
+  const int c64 = n < 64 ? n : 64;
+#pragma unroll 8
+  for (int k = 0; k < c64; k++) {
+    const float a0 = lane > k && own0 ? r0[k] : 0.0f, a1 = own1 ? r1[k] : 0.0f;
+    const float yk = lane_value(div_by(y0, l0, v0), k);
+    if (lane == k) y0 = yk;
+    else if (lane > k) y0 = fmaf(-a0, yk, y0);
+    y1 = fmaf(-a1, yk, y1);
+  }
+#pragma unroll 8
+  for (int k = 64; k < n; k++) {
+    const float a1 = i1 > k && own1 ? r1[k] : 0.0f;
+    const float yk = lane_value(div_by(y1, l1, v1), k - 64);
+    if (i1 == k) y1 = yk;
+    else if (i1 > k) y1 = fmaf(-a1, yk, y1);
+  }
+#pragma unroll 8
+  for (int k = n - 1; k >= 64; k--) {
+    const float* const row = A + tri_row(k);
+    const float a0 = row[lane], a1 = i1 < k ? row[i1] : 0.0f;
+    const float xk = lane_value(div_by(y1, l1, v1), k - 64);
+    if (i1 == k) y1 = xk;
+    else if (i1 < k) y1 = fmaf(-a1, xk, y1);
+    y0 = fmaf(-a0, xk, y0);
+  }
+#pragma unroll 8
+  for (int k = c64 - 1; k >= 0; k--) {
+    const float a0 = lane < k ? A[tri_row(k) + lane] : 0.0f;
+    const float xk = lane_value(div_by(y0, l0, v0), k);
+    if (lane == k) y0 = xk;
+    else if (lane < k) y0 = fmaf(-a0, xk, y0);
+  }
+  *x0 = y0;
+  *x1 = y1;
+}
+
+// The lower triangle f(row, column) into packed A, and a factor from packed A
+// into the block L (row stride ld) with zeros above the diagonal.
+// Rows are taken nine at a time, their loads in flight together (lanes past a
+// row's end load its last entry, so that no load waits in a branch).
+template <class F>
+MJH_DEV void tri_load(float* A, int n, int lane, F f) {
+  constexpr int U = 9;
+  for (int s = 0; s < n; s += 64) {
+    const int c = lane + s;
+    for (int r0 = s; r0 < n; r0 += U) {
+      float v[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int r = min(r0 + u, n - 1);
+        v[u] = f(r, min(c, r));
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (r0 + u < n && c <= r0 + u) A[tri_row(r0 + u) + c] = v[u];
+    }
+  }
+  wave_fence();
+}
+MJH_DEV void tri_store(const float* A, int n, float* L, int ld, int lane) {
+  for (int c = lane; c < n; c += 64) {
+#pragma unroll 9
+    for (int r = 0; r < n; r++) {
+      const float v = A[tri_row(r) + min(c, r)];
+      L[r * ld + c] = c <= r ? v : 0.0f;
+    }
+  }
+}
+// x = inv(A) b for one block, given its lower triangle by f and what its
+// diagonal gains by diag(entry, row); A: n (n + 1) / 2 floats of LDS; factored:
+// f gives the factor.
+template <class F, class G, class B, class X>
+MJH_DEV void tri_solve(float* A, int n, int lane, bool factored, F f, G diag, B b, X x) {
+  tri_load(A, n, lane, f);
+  for (int i = lane; i < n; i += 64) diag(A[tri_row(i) + i], i);
+  float x0 = lane < n ? b(lane) : 0.0f, x1 = lane + 64 < n ? b(lane + 64) : 0.0f;
+  if (!factored) chol_tri(A, n, lane);
+  cho_solve_tri(A, n, &x0, &x1, lane);
+  if (lane < n) x(lane, x0);
+  if (lane + 64 < n) x(lane + 64, x1);
+  sync();
+}
+
 // Factor the tree blocks of M (global, [nv, nv]) into L (global, may alias
-// a different array) through an LDS staging buffer of nv*nv floats.
+// a different array) through an LDS staging buffer of nv*nv floats.  64-lane
+// teams take the blocks up to kTriMax packed (chol_tri), the same bits with no
+// barrier a column: factor_m and the integrator of three attached humanoids,
+// 1024 worlds, 146 and 180 us to 86 and 107.
 template <int TEAM>
 MJH_DEV void factor_blocks(const mjhModel& m, const float* M, float* L, float* lds, const Team<TEAM>& t) {
   if constexpr (TEAM == kRegTeam) {
@@ -542,6 +788,14 @@ MJH_DEV void factor_blocks(const mjhModel& m, const float* M, float* L, float* l
   }
   const int nv = m.nv;
   for_each_tree_block(m, [&](int dof, int n) {
+    if (TEAM == 64 && n <= kTriMax) {
+      const float* const Mb = M + dof * nv + dof;
+      tri_load(lds, n, t.lane, [&](int r, int c) { return Mb[r * nv + c]; });
+      chol_tri(lds, n, t.lane);
+      tri_store(lds, n, L + dof * nv + dof, nv, t.lane);
+      sync();
+      return;
+    }
     for (int p = t.lane; p < n * n; p += TEAM) lds[p] = M[(dof + p / n) * nv + dof + p % n];
     sync();
     chol_lds(lds, n, n, m, t);
@@ -561,6 +815,12 @@ MJH_DEV void solve_blocks(const mjhModel& m, const float* L, float* x, const flo
   }
   const int nv = m.nv;
   for_each_tree_block(m, [&](int dof, int n) {
+    if (TEAM == 64 && n <= kTriMax) {
+      const float* const Lb = L + dof * nv + dof;
+      tri_solve(lds, n, t.lane, true, [&](int r, int c) { return Lb[r * nv + c]; }, [](float&, int) {},
+                [&](int i) { return y[dof + i]; }, [&](int i, float v) { x[dof + i] = v; });
+      return;
+    }
     float* Ls = lds;
     float* xs = lds + n * n;
     for (int p = t.lane; p < n * n; p += TEAM) Ls[p] = L[(dof + p / n) * nv + dof + p % n];
@@ -574,7 +834,7 @@ MJH_DEV void solve_blocks(const mjhModel& m, const float* L, float* x, const flo
 
 // smooth.py:383-395 factor_m: the dense Cholesky factor qLDd of qMd, and
 // for sparse models MuJoCo's L'DL factor of qM into qLD / qLDiagInv.
-// lds: nv * nv floats (at least nM).
+// lds: nv * nv floats (at least lds_sparse_words).
 template <int TEAM>
 MJH_DEV void factor_m(const mjhModel& m, const mjhData& d, float* lds, const Team<TEAM>& t) {
   const int nv = m.nv, w = t.world;

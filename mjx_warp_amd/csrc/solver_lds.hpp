@@ -26,7 +26,6 @@ constexpr int kFlagDeferred = 1;
 // in efc_h with the blocked Cholesky's panel buffer in LDS; kHessTri, its
 // lower triangle packed by rows in LDS, two rows per lane (nv <= kTriMax).
 enum { kHessSquare = 0, kHessGlobal = 1, kHessTri = 2 };
-constexpr int kTriMax = 128;
 
 // LDS floats per world: the Hessian (or its panel buffer) + 14 nv (vectors) +
 // 8 rmax (rows) + rj nv (staged Jacobian rows).  The mass
@@ -34,140 +33,6 @@ constexpr int kTriMax = 128;
 __host__ __device__ inline int lds_solver_floats(int nv, int rmax, int rj, int hess = kHessSquare) {
   const int h = hess == kHessGlobal ? chol_blocked_floats(nv) : hess == kHessTri ? nv * (nv + 1) / 2 : nv * nv;
   return h + 14 * nv + 8 * rmax + rj * nv;
-}
-
-MJH_DEV int tri_row(int i) { return i * (i + 1) / 2; }
-MJH_DEV float lane_value(float v, int k) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
-}
-
-// Cholesky factor of the packed lower triangle A (n <= kTriMax) by one
-// 64-lane team, in place.  Lane l owns rows l and l + 64, and nobody else
-// touches them: a panel of kTriPanel columns is factored with the rows'
-// entries in registers, the diagonal rows' read by readlane, and the rows'
-// later entries then take the panel's products column by column, the column's
-// row of the panel read by readlane as well -- no barrier and no LDS word
-// shared between lanes (row starts are triangular numbers, distinct modulo
-// the banks).  Each entry gets the operations of chol_lds in its order, so
-// the factor is the same bit for bit.  Bound by the serial chain of square
-// root, reciprocal and broadcasts down the diagonal, where chol_lds passes
-// every column through LDS with three barriers (170 us at nv 81) and
-// chol_blocked goes to efc_h in global memory (205 us): 1024 worlds of three
-// attached humanoids step in 2.23 ms with it, 4.53 ms before.
-constexpr int kTriPanel = 16;
-// One panel from column p on: r0, r1 the lane's rows.  kHigh: the panel's
-// diagonal rows are the lanes' second rows (p >= 64), the first are done.
-// Columns past n work on zeros (and what comes of them), which nobody keeps.
-template <bool kHigh>
-MJH_DEV void chol_tri_panel(float* r0, float* r1, int n, int p, int lane) {
-  constexpr int B = kTriPanel;
-  const int i1 = lane + 64, q0 = kHigh ? p - 64 : p;  // the lane of the first diagonal row
-  const bool own0 = !kHigh && lane < n, own1 = i1 < n;
-  float x0[B], x1[B];
-#pragma unroll
-  for (int k = 0; k < B; k++) {
-    x0[k] = own0 && lane >= p + k ? r0[p + k] : 0.0f;
-    x1[k] = own1 && i1 >= p + k ? r1[p + k] : 0.0f;
-  }
-#pragma unroll
-  for (int k = 0; k < B; k++) {
-    const float dkk = sqrtf(lane_value(kHigh ? x1[k] : x0[k], q0 + k));
-    const float inv = 1.0f / dkk;
-    if (!kHigh) x0[k] = lane == q0 + k ? dkk : x0[k] * inv;
-    x1[k] = kHigh && lane == q0 + k ? dkk : x1[k] * inv;
-#pragma unroll
-    for (int j = k + 1; j < B; j++) {
-      const float l = lane_value(kHigh ? x1[k] : x0[k], q0 + j);
-      if (!kHigh) x0[j] = fmaf(-x0[k], l, x0[j]);
-      x1[j] = fmaf(-x1[k], l, x1[j]);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < B; k++) {
-    if (own0 && lane >= p + k) r0[p + k] = x0[k];
-    if (own1 && i1 >= p + k) r1[p + k] = x1[k];
-  }
-  int c = p + B;
-  if (!kHigh) {
-    const int c64 = n < 64 ? n : 64;
-#pragma unroll 2
-    for (; c < c64; c++) {
-      const bool u0 = own0 && lane >= c;
-      float a0 = u0 ? r0[c] : 0.0f, a1 = own1 ? r1[c] : 0.0f;
-#pragma unroll
-      for (int k = 0; k < B; k++) {
-        const float l = lane_value(x0[k], c);
-        a0 = fmaf(-x0[k], l, a0);
-        a1 = fmaf(-x1[k], l, a1);
-      }
-      if (u0) r0[c] = a0;
-      if (own1) r1[c] = a1;
-    }
-  }
-#pragma unroll 2
-  for (; c < n; c++) {
-    const bool u1 = own1 && i1 >= c;
-    float a1 = u1 ? r1[c] : 0.0f;
-#pragma unroll
-    for (int k = 0; k < B; k++) a1 = fmaf(-x1[k], lane_value(x1[k], c - 64), a1);
-    if (u1) r1[c] = a1;
-  }
-}
-MJH_DEV void chol_tri(float* A, int n, int lane) {
-  static_assert(64 % kTriPanel == 0, "a panel's diagonal rows are one set of rows");
-  float* const r0 = A + tri_row(lane < n ? lane : 0);
-  float* const r1 = A + tri_row(lane + 64 < n ? lane + 64 : 0);
-#pragma unroll 1
-  for (int p = 0; p < n && p < 64; p += kTriPanel) chol_tri_panel<false>(r0, r1, n, p, lane);
-#pragma unroll 1
-  for (int p = 64; p < n; p += kTriPanel) chol_tri_panel<true>(r0, r1, n, p, lane);
-  wave_fence();
-}
-
-// x = inv(L L') x for the packed factor, x one entry per lane and set (lanes
-// l and l + 64); each entry gets the operations of cho_solve_wave in its
-// order.  The rows' words do not depend on the chain and are loaded ahead.
-MJH_DEV void cho_solve_tri(const float* A, int n, float* x0, float* x1, int lane) {
-  const int i1 = lane + 64;
-  const bool own0 = lane < n, own1 = i1 < n;
-  const float* const r0 = A + tri_row(own0 ? lane : 0);
-  const float* const r1 = A + tri_row(own1 ? i1 : 0);
-  const float l0 = own0 ? r0[lane] : 1.0f, l1 = own1 ? r1[i1] : 1.0f;
-  float y0 = own0 ? *x0 : 0.0f, y1 = own1 ? *x1 : 0.0f;
-  const int c64 = n < 64 ? n : 64;
-#pragma unroll 8
-  for (int k = 0; k < c64; k++) {
-    const float a0 = lane > k && own0 ? r0[k] : 0.0f, a1 = own1 ? r1[k] : 0.0f;
-    const float yk = lane_value(y0 / l0, k);
-    if (lane == k) y0 = yk;
-    else if (lane > k) y0 = fmaf(-a0, yk, y0);
-    y1 = fmaf(-a1, yk, y1);
-  }
-#pragma unroll 8
-  for (int k = 64; k < n; k++) {
-    const float a1 = i1 > k && own1 ? r1[k] : 0.0f;
-    const float yk = lane_value(y1 / l1, k - 64);
-    if (i1 == k) y1 = yk;
-    else if (i1 > k) y1 = fmaf(-a1, yk, y1);
-  }
-#pragma unroll 8
-  for (int k = n - 1; k >= 64; k--) {
-    const float* const row = A + tri_row(k);
-    const float a0 = row[lane], a1 = i1 < k ? row[i1] : 0.0f;
-    const float xk = lane_value(y1 / l1, k - 64);
-    if (i1 == k) y1 = xk;
-    else if (i1 < k) y1 = fmaf(-a1, xk, y1);
-    y0 = fmaf(-a0, xk, y0);
-  }
-#pragma unroll 8
-  for (int k = c64 - 1; k >= 0; k--) {
-    const float a0 = lane < k ? A[tri_row(k) + lane] : 0.0f;
-    const float xk = lane_value(y0 / l0, k);
-    if (lane == k) y0 = xk;
-    else if (lane < k) y0 = fmaf(-a0, xk, y0);
-  }
-  *x0 = y0;
-  *x1 = y1;
 }
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));

@@ -1,0 +1,63 @@
+"""Mass-matrix factors on 64-lane teams: the packed blocks (one row a lane, two
+rows, the largest packed and the first that is not) and the sparse L'DL factor
+(its look-up table in LDS, also on 32-lane teams, more ancestors than a pass
+takes, and a matrix too large for the table), against float32 backward error
+bounds: |M x - b| <= g |L| |L'| |x| and |M - L' D L| <= g |L'| |D| |L|, with
+g = 4 (3 n + 4) eps and 4 (n + 4) eps (the textbook constants times 4)."""
+import numpy as np
+import pytest
+import torch
+
+import helpers
+import mjx_warp_amd as mjw
+from mjx_warp_amd import models
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(np.float32).eps
+
+
+@pytest.mark.parametrize("nv", [33, 64, 65, 81, 128, 129])
+def test_packed_blocks(nv):
+  mjm = models.chain(nv)
+  m = mjw.put_model(mjm)
+  d = mjw.make_data(mjm, nworld=2, nconmax=16, njmax=4 * nv)
+  rng = np.random.default_rng(nv)
+  A = rng.normal(size=(2, nv, nv))
+  M = (A @ A.transpose(0, 2, 1) + nv * np.eye(nv)).astype(np.float32)
+  b = rng.normal(size=(2, nv)).astype(np.float32)
+  field = "qMd" if m.opt.is_sparse else "qM"
+  helpers.set_field(d, field, M)
+  mjw.factor_m(m, d)
+  x = torch.zeros(2, nv, device="cuda")
+  mjw.solve_m(m, d, x, torch.as_tensor(b, device="cuda"))
+  torch.cuda.synchronize()
+  for w in range(2):
+    H, y = M[w].astype(np.float64), x[w].cpu().numpy().astype(np.float64)
+    L = np.abs(np.linalg.cholesky(H))
+    assert np.all(np.abs(H @ y - b[w]) <= 4 * (3 * nv + 4) * EPS * (L @ (L.T @ np.abs(y))))
+
+
+@pytest.mark.parametrize("nv", [2, 17, 32, 33, 60, 126, 128])
+def test_sparse_factor(nv):
+  mjm = models.chain(nv)
+  mjm.opt.jacobian = 1
+  m = mjw.put_model(mjm)
+  assert m.opt.is_sparse
+  d = mjw.make_data(mjm, nworld=3, nconmax=48, njmax=12 * nv)
+  rng = np.random.default_rng(nv)
+  helpers.set_field(d, "qpos", rng.uniform(-0.3, 0.3, (3, nv)))
+  mjw.kinematics(m, d)
+  mjw.com_pos(m, d)
+  mjw.crb(m, d)
+  mjw.factor_m(m, d)
+  torch.cuda.synchronize()
+  # a chain: row i of the sparse layout is M(i, i), M(i, i - 1), ...
+  rows = lambda a: [np.pad(r[::-1], (0, nv - len(r))) for r in np.split(a, np.cumsum(np.arange(1, nv)))]
+  S, F = (helpers.data_numpy(d, k).reshape(3, -1).astype(np.float64) for k in ("qM", "qLD"))
+  inv = helpers.data_numpy(d, "qLDiagInv").reshape(3, nv)
+  for w in range(3):
+    T, U = np.array(rows(S[w])), np.array(rows(F[w]))
+    M = T + np.tril(T, -1).T
+    D, L = np.diag(U).copy(), np.tril(U, -1) + np.eye(nv)
+    assert np.all(np.abs(M - L.T @ (D[:, None] * L)) <= 4 * (nv + 4) * EPS * (np.abs(L.T) @ (np.abs(D)[:, None] * np.abs(L))))
+    assert np.allclose(inv[w] * D, 1, rtol=0, atol=2 * EPS)
