@@ -576,6 +576,9 @@ int reset(const mjhData& d, hipStream_t s, int which) {
 
 
 
+// Whether the sweep-and-prune stages run kSapWaves wavefronts a world: every
+// model over 100 geoms, in batches whose threads a grid can count.
+bool pair_waves(const mjhModel& m, const mjhData& d) { return m.ngeom > 100 && d.nworld <= (1 << 22); }
 // A stage of sweep-and-prune collision, kSapWaves wavefronts a world.
 template <class S>
 int launch_waves(const mjhModel& m, const mjhData& d, hipStream_t s, int words, const char* name) {
@@ -587,11 +590,12 @@ int launch_waves(const mjhModel& m, const mjhData& d, hipStream_t s, int words, 
 }
 
 int do_collision(const mjhModel& m, const mjhData& d, hipStream_t s) {
-  if (m.ngeom > 100) {
+  if (pair_waves(m, d)) {
     TRY(launch_waves<StSapWaves>(m, d, s, lds_sap(m), "broadphase"));
     return launch_waves<StNarrowWaves>(m, d, s, kNarrowWords, "narrowphase");
   }
-  TRY(launch<StNxn>(m, d, s, lds_broadphase(m), "broadphase"));
+  if (m.ngeom > 100) TRY(launch<StSap>(m, d, s, lds_sap(m), "broadphase"));
+  else TRY(launch<StNxn>(m, d, s, lds_broadphase(m), "broadphase"));
   return launch<StNarrowphase>(m, d, s, 0, "narrowphase");
 }
 
@@ -1089,11 +1093,11 @@ int mjh_nxn_broadphase(const mjhModel* m, const mjhData* d, mjhStream stream) {
 }
 int mjh_sap_broadphase(const mjhModel* m, const mjhData* d, mjhStream stream) {
   TRY(reset(*d, (hipStream_t)stream, 1));
-  if (m->ngeom > 100) return launch_waves<StSapWaves>(*m, *d, (hipStream_t)stream, lds_sap(*m), "sap_broadphase");
+  if (pair_waves(*m, *d)) return launch_waves<StSapWaves>(*m, *d, (hipStream_t)stream, lds_sap(*m), "sap_broadphase");
   return launch<StSap>(*m, *d, (hipStream_t)stream, lds_sap(*m), "sap_broadphase");
 }
 int mjh_primitive_narrowphase(const mjhModel* m, const mjhData* d, mjhStream stream) {
-  if (m->ngeom > 100)
+  if (pair_waves(*m, *d))
     return launch_waves<StNarrowWaves>(*m, *d, (hipStream_t)stream, kNarrowWords, "primitive_narrowphase");
   return launch<StNarrowphase>(*m, *d, (hipStream_t)stream, 0, "primitive_narrowphase");
 }

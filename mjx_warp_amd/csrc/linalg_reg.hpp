@@ -44,11 +44,17 @@ MJH_DEV void wave_fence() {
 // the others.  The mask is two scalar moves at its use, where a comparison
 // with the lane number is a vector instruction for each column, and masks that
 // the compiler knows of leave a loop for scalar registers that it then spills.
-template <unsigned MASK>
+// kDpp: the result is a DPP operand, read two wait states after the write at the
+// earliest (the compiler keeps that distance for its own instructions only).
+template <unsigned MASK, bool kDpp = false>
 MJH_DEV float pick(float yes, float no) {
   float r;
-  asm("s_mov_b32 vcc_lo, %3\n\ts_mov_b32 vcc_hi, vcc_lo\n\tv_cndmask_b32_e32 %0, %1, %2, vcc"
-      : "=v"(r) : "v"(no), "v"(yes), "i"(MASK) : "vcc");
+  if constexpr (kDpp)
+    asm("s_mov_b32 vcc_lo, %3\n\ts_mov_b32 vcc_hi, vcc_lo\n\tv_cndmask_b32_e32 %0, %1, %2, vcc\n\ts_nop 1"
+        : "=v"(r) : "v"(no), "v"(yes), "i"(MASK) : "vcc");
+  else
+    asm("s_mov_b32 vcc_lo, %3\n\ts_mov_b32 vcc_hi, vcc_lo\n\tv_cndmask_b32_e32 %0, %1, %2, vcc"
+        : "=v"(r) : "v"(no), "v"(yes), "i"(MASK) : "vcc");
   return r;
 }
 // lane k, and the lanes past k
@@ -332,21 +338,21 @@ struct RegChol {
     for (int i = 0; i < 8; i++) {  // columns 2 i, 2 i + 1; the first has bit 0 ^ bit 2 = (i >> 1) & 1
       const int f = (i >> 1) & 1;
       const float lo = a[2 * i + f], hi = a[2 * i + 1 - f];
-      b[i] = pick<m1>(hi, lo) + dpp_f<0xB1>(pick<m1>(lo, hi));
+      b[i] = pick<m1>(hi, lo) + dpp_f<0xB1>(pick<m1, true>(lo, hi));
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {  // b[2 i], b[2 i + 1] are columns 4 i.. and 4 i + 2..
       const int f = i & 1;
       const float lo = b[2 * i + f], hi = b[2 * i + 1 - f];
-      c[i] = pick<m2>(hi, lo) + dpp_f<0x4E>(pick<m2>(lo, hi));
+      c[i] = pick<m2>(hi, lo) + dpp_f<0x4E>(pick<m2, true>(lo, hi));
     }
 #pragma unroll
     for (int i = 0; i < 2; i++) {  // c[2 i], c[2 i + 1] are columns 8 i.. and 8 i + 4..
       const int f = i;
       const float lo = c[2 * i + f], hi = c[2 * i + 1 - f];
-      e[i] = pick<m3>(hi, lo) + dpp_f<0x141>(pick<m3>(lo, hi));
+      e[i] = pick<m3>(hi, lo) + dpp_f<0x141>(pick<m3, true>(lo, hi));
     }
-    return pick<m4>(e[1], e[0]) + dpp_f<0x140>(pick<m4>(e[0], e[1]));
+    return pick<m4>(e[1], e[0]) + dpp_f<0x140>(pick<m4, true>(e[0], e[1]));
   }
 
   // Writes the rows into the blocks [beg, end) of A (global, [nv, nv]) by
