@@ -407,42 +407,20 @@ MJH_DEV void euler(const mjhModel& m, const mjhData& d, float* lds, const Team<T
   if (m.opt.is_sparse) euler_sparse_outputs(m, d, lds, t);
   if constexpr (TEAM == kRegTeam) {
     integrate_reg(m, d, true, lds, t);
-    return;
+  } else {
+    if (t.valid) {
+      const float* qM = WPTR(d.qMd, w, nv * nv);
+      const float* qs = WPTR(d.qfrc_smooth, w, nv);
+      const float* qc = WPTR(d.qfrc_constraint, w, nv);
+      float* qacc_int = WPTR(d.qacc_integration, w, nv);
+      const float dt = m.opt.timestep;
+      solve_tree_blocks(m, lds, t, false, qM, [&](float& v, int i) { v += m.dof_damping[i] * dt; },
+                        [&](int i) { return qs[i] + qc[i]; }, [&](int i, float v) { qacc_int[i] = v; });
+    }
+    sync();
+    advance(m, d, d.qacc_integration, t);
+    sync();
   }
-  if (t.valid) {
-    const float* qM = WPTR(d.qMd, w, nv * nv);
-    const float* qs = WPTR(d.qfrc_smooth, w, nv);
-    const float* qc = WPTR(d.qfrc_constraint, w, nv);
-    float* qacc_int = WPTR(d.qacc_integration, w, nv);
-    const float dt = m.opt.timestep;
-    for_each_tree_block(m, [&](int dof, int n) {
-      if (n <= kTriMax) {
-        const float* const Mb = qM + dof * nv + dof;
-        tri_solve(lds, n, t.lane, false,
-                  [&](int r, int c) { return Mb[r * nv + c]; },
-                  [&](float& v, int i) { v += m.dof_damping[dof + i] * dt; },
-                  [&](int i) { return qs[dof + i] + qc[dof + i]; }, [&](int i, float v) { qacc_int[dof + i] = v; });
-        return;
-      }
-      float* A = lds;
-      float* x = lds + n * n;
-      for (int p = t.lane; p < n * n; p += TEAM) {
-        const int r = p / n, c = p % n;
-        float v = qM[(dof + r) * nv + dof + c];
-        if (r == c) v += m.dof_damping[dof + r] * dt;
-        A[p] = v;
-      }
-      for (int p = t.lane; p < n; p += TEAM) x[p] = qs[dof + p] + qc[dof + p];
-      sync();
-      chol_lds(A, n, n, m, t);
-      cho_solve_lds(A, n, n, x, t);
-      for (int p = t.lane; p < n; p += TEAM) qacc_int[dof + p] = x[p];
-      sync();
-    });
-  }
-  sync();
-  advance(m, d, d.qacc_integration, t);
-  sync();
 }
 
 // forward.py:245-405 implicit (implicitfast, dense); lds: nv*nv + nv floats
@@ -491,23 +469,9 @@ MJH_DEV void implicit(const mjhModel& m, const mjhData& d, float* lds, const Tea
     const float* qMi = WPTR(d.qM_integration, w, nv * nv);
     const float* qfi = WPTR(d.qfrc_integration, w, nv);
     float* qacc_int = WPTR(d.qacc_integration, w, nv);
-    for_each_tree_block(m, [&](int dof, int n) {
-      if (n <= kTriMax) {
-        const float* const Mb = qMi + dof * nv + dof;
-        tri_solve(lds, n, t.lane, false, [&](int r, int c) { return Mb[r * nv + c]; }, [](float&, int) {},
-                  [&](int i) { return qfi[dof + i]; }, [&](int i, float v) { qacc_int[dof + i] = v; });
-        return;
-      }
-      float* A = lds;
-      float* x = lds + n * n;
-      for (int p = t.lane; p < n * n; p += TEAM) A[p] = qMi[(dof + p / n) * nv + dof + p % n];
-      for (int p = t.lane; p < n; p += TEAM) x[p] = qfi[dof + p];
-      sync();
-      chol_lds(A, n, n, m, t);
-      cho_solve_lds(A, n, n, x, t);
-      for (int p = t.lane; p < n; p += TEAM) qacc_int[dof + p] = x[p];
-      sync();
-    });
+    if constexpr (TEAM == 64)
+      solve_tree_blocks(m, lds, t, false, qMi, [](float&, int) {}, [&](int i) { return qfi[i]; },
+                        [&](int i, float v) { qacc_int[i] = v; });
   }
   sync();
   advance(m, d, d.qacc_integration, t);

@@ -597,13 +597,12 @@ MJH_DEV float lane_value(float v, int k) {
 // chol_blocked goes to efc_h in global memory (205 us): 1024 worlds of three
 // attached humanoids step in 2.23 ms with it, 4.53 ms before.
 constexpr int kTriPanel = 16;
-// One panel from column p on: r0, r1 the lane's rows.  kHigh: the panel's
+// One panel of B columns from column p on: r0, r1 the lane's rows.  kHigh: the panel's
 // diagonal rows are the lanes' second rows (p >= 64), the first are done.
 // Columns past n work on zeros (and what comes of them), which nobody keeps.
 // kTwo unset: n <= 64, no second rows.
-template <bool kHigh, bool kTwo>
+template <bool kHigh, bool kTwo, int B>
 MJH_DEV void chol_tri_panel(float* r0, float* r1, int n, int p, int lane) {
-  constexpr int B = kTriPanel;
   const int i1 = lane + 64, q0 = kHigh ? p - 64 : p;  // the lane of the first diagonal row
   const bool own0 = !kHigh && lane < n, own1 = kTwo && i1 < n;
   float x0[B], x1[B];
@@ -662,12 +661,29 @@ MJH_DEV void chol_tri(float* A, int n, int lane) {
   float* const r1 = A + tri_row(lane + 64 < n ? lane + 64 : 0);
   if (n <= 64) {
 #pragma unroll 1
-    for (int p = 0; p < n; p += kTriPanel) chol_tri_panel<false, false>(r0, r1, n, p, lane);
+    for (int p = 0; p < n; p += kTriPanel) chol_tri_panel<false, false, kTriPanel>(r0, r1, n, p, lane);
   } else {
 #pragma unroll 1
-    for (int p = 0; p < 64; p += kTriPanel) chol_tri_panel<false, true>(r0, r1, n, p, lane);
+    for (int p = 0; p < 64; p += kTriPanel) chol_tri_panel<false, true, kTriPanel>(r0, r1, n, p, lane);
 #pragma unroll 1
-    for (int p = 64; p < n; p += kTriPanel) chol_tri_panel<true, true>(r0, r1, n, p, lane);
+    for (int p = 64; p < n; p += kTriPanel) chol_tri_panel<true, true, kTriPanel>(r0, r1, n, p, lane);
+  }
+  wave_fence();
+}
+// A tree's block past kTinyMax: a panel wider than the block works its columns
+// past the block on zeros, and with few real columns that is most of the time,
+// so blocks up to 12 take panels of 8 (where one does) or 6.  factor_m of 8192
+// worlds in us, blocks in LDS (chol_lds) / packed with panels of 16 / as here:
+// ten of 8 111 / 168 / 94, eight of 9 116 / 138 / 99, six of 12 133 / 116 / 95,
+// six of 13 149 / 118 / 118.
+MJH_DEV void chol_tri_block(float* A, int n, int lane) {
+  if (n > 12) return chol_tri(A, n, lane);
+  float* const r0 = A + tri_row(lane < n ? lane : 0);
+  if (n <= 8) {
+    chol_tri_panel<false, false, 8>(r0, A, n, 0, lane);
+  } else {
+#pragma unroll 1
+    for (int p = 0; p < n; p += 6) chol_tri_panel<false, false, 6>(r0, A, n, p, lane);
   }
   wave_fence();
 }
@@ -760,6 +776,74 @@ MJH_DEV void tri_store(const float* A, int n, float* L, int ld, int lane) {
     }
   }
 }
+// ---- blocks of at most kTinyMax dofs: a lane takes a whole tree's, in
+// registers, with the operations of chol_lds and cho_solve_lds on each entry.
+// Bound by the loads' latency; a team per tree left most lanes idle through
+// every square root and division.  factor_m / solve_m / euler of 8192 worlds in
+// us, a block at a time in LDS and as here: forty of 1 dof 76 / 71 / 136 and
+// 12 / 9 / 15, twenty of 6 161 / 94 / 249 and 58 / 23 / 33.  Up to 8 dofs the
+// registers would take a wavefront per SIMD from solve_m (eight blocks of 9: 56
+// us, 48 so).
+constexpr int kTinyMax = 6;
+struct TinyBlock {
+  float a[kTinyMax * (kTinyMax + 1) / 2], y[kTinyMax];
+  static constexpr int at(int r, int c) { return r * (r + 1) / 2 + c; }
+  template <class F>
+  MJH_DEV void load(int n, F f) {
+#pragma unroll
+    for (int r = 0; r < kTinyMax; r++)
+#pragma unroll
+      for (int c = 0; c <= r; c++) a[at(r, c)] = r < n ? f(r, c) : 0.0f;
+  }
+  MJH_DEV void factor(int n) {
+#pragma unroll
+    for (int k = 0; k < kTinyMax; k++) {
+      if (k >= n) break;
+      const float dkk = sqrtf(a[at(k, k)]);
+      const float inv = 1.0f / dkk;
+      a[at(k, k)] = dkk;
+#pragma unroll
+      for (int i = k + 1; i < kTinyMax; i++) a[at(i, k)] *= inv;
+#pragma unroll
+      for (int i = k + 1; i < kTinyMax; i++)
+#pragma unroll
+        for (int j = k + 1; j <= i; j++) a[at(i, j)] = fmaf(-a[at(i, k)], a[at(j, k)], a[at(i, j)]);
+    }
+  }
+  // y becomes inv(L L') y
+  MJH_DEV void solve(int n) {
+#pragma unroll
+    for (int k = 0; k < kTinyMax; k++) {
+      if (k >= n) break;
+      y[k] = y[k] / a[at(k, k)];
+#pragma unroll
+      for (int i = k + 1; i < kTinyMax; i++) y[i] = fmaf(-a[at(i, k)], y[k], y[i]);
+    }
+#pragma unroll
+    for (int k = kTinyMax - 1; k >= 0; k--) {
+      if (k >= n) continue;
+      y[k] = y[k] / a[at(k, k)];
+#pragma unroll
+      for (int i = 0; i < k; i++) y[i] = fmaf(-a[at(k, i)], y[k], y[i]);
+    }
+  }
+};
+// for_each_tree_block on a 64-lane team, the trees of at most kTinyMax dofs
+// handed out a tree per lane: f(dof, size, whether by the lane alone).
+template <class F>
+MJH_DEV void for_each_sized_block(const mjhModel& m, int lane, F f) {
+  for (int g = 0; g < m.nqLD_group; g++) {
+    const int beg = m.qLD_tileadr[g], size = m.qLD_tilesize[g];
+    const int end = (g == m.nqLD_group - 1) ? m.nqLD_tile : m.qLD_tileadr[g + 1];
+    if (size <= kTinyMax) {
+      for (int k = beg + lane; k < end; k += 64) f(m.qLD_tile[k], size, std::true_type{});
+      sync();
+      continue;
+    }
+    for (int k = beg; k < end; k++) f(m.qLD_tile[k], size, std::false_type{});
+  }
+}
+
 // x = inv(A) b for one block, given its lower triangle by f and what its
 // diagonal gains by diag(entry, row); A: n (n + 1) / 2 floats of LDS; factored:
 // f gives the factor.
@@ -768,17 +852,68 @@ MJH_DEV void tri_solve(float* A, int n, int lane, bool factored, F f, G diag, B 
   tri_load(A, n, lane, f);
   for (int i = lane; i < n; i += 64) diag(A[tri_row(i) + i], i);
   float x0 = lane < n ? b(lane) : 0.0f, x1 = lane + 64 < n ? b(lane + 64) : 0.0f;
-  if (!factored) chol_tri(A, n, lane);
+  if (!factored) chol_tri_block(A, n, lane);
   cho_solve_tri(A, n, &x0, &x1, lane);
   if (lane < n) x(lane, x0);
   if (lane + 64 < n) x(lane + 64, x1);
   sync();
 }
 
+// ... for one tree of at most kTinyMax dofs, by the calling lane
+template <class F, class G, class B, class X>
+MJH_DEV void tiny_solve(int n, bool factored, F f, G diag, B b, X x) {
+  TinyBlock T;
+  T.load(n, f);
+#pragma unroll
+  for (int i = 0; i < kTinyMax; i++) {
+    if (i < n) diag(T.a[T.at(i, i)], i);
+    T.y[i] = i < n ? b(i) : 0.0f;
+  }
+  if (!factored) T.factor(n);
+  T.solve(n);
+#pragma unroll
+  for (int i = 0; i < kTinyMax; i++)
+    if (i < n) x(i, T.y[i]);
+}
+// x = inv(A) b for every tree block of a 64-lane team's world: A global
+// [nv, nv] (factored: the factor's blocks), its diagonal's gain diag(entry, i),
+// b(i) and x(i, value) by dof; lds: n n + n floats of the largest block.
+template <class G, class B, class X>
+MJH_DEV void solve_tree_blocks(const mjhModel& m, float* lds, const Team<64>& t, bool factored, const float* A, G diag,
+                               B b, X x) {
+  const int nv = m.nv;
+  for_each_sized_block(m, t.lane, [&](int dof, int n, auto tiny) {
+    const float* const Ab = A + dof * nv + dof;
+    auto Af = [&](int r, int c) { return Ab[r * nv + c]; };
+    auto dg = [&](float& v, int i) { diag(v, dof + i); };
+    auto bf = [&](int i) { return b(dof + i); };
+    auto xf = [&](int i, float v) { x(dof + i, v); };
+    if constexpr (decltype(tiny)::value) {
+      tiny_solve(n, factored, Af, dg, bf, xf);
+    } else if (n <= kTriMax) {
+      tri_solve(lds, n, t.lane, factored, Af, dg, bf, xf);
+    } else {
+      float* const M = lds;
+      float* const y = lds + n * n;
+      for (int p = t.lane; p < n * n; p += 64) {
+        float v = Af(p / n, p % n);
+        if (p / n == p % n) dg(v, p / n);
+        M[p] = v;
+      }
+      for (int i = t.lane; i < n; i += 64) y[i] = bf(i);
+      sync();
+      if (!factored) chol_lds(M, n, n, m, t);
+      cho_solve_lds(M, n, n, y, t);
+      for (int i = t.lane; i < n; i += 64) xf(i, y[i]);
+      sync();
+    }
+  });
+}
+
 // Factor the tree blocks of M (global, [nv, nv]) into L (global, may alias
 // a different array) through an LDS staging buffer of nv*nv floats.  64-lane
-// teams take the blocks up to kTriMax packed (chol_tri), the same bits with no
-// barrier a column: factor_m and the integrator of three attached humanoids,
+// teams take the blocks up to kTriMax packed (chol_tri_block), the same bits
+// with no barrier a column: factor_m and the integrator of three attached humanoids,
 // 1024 worlds, 146 and 180 us to 86 and 107.
 template <int TEAM>
 MJH_DEV void factor_blocks(const mjhModel& m, const float* M, float* L, float* lds, const Team<TEAM>& t) {
@@ -787,20 +922,30 @@ MJH_DEV void factor_blocks(const mjhModel& m, const float* M, float* L, float* l
     return;
   }
   const int nv = m.nv;
-  for_each_tree_block(m, [&](int dof, int n) {
-    if (TEAM == 64 && n <= kTriMax) {
-      const float* const Mb = M + dof * nv + dof;
+  for_each_sized_block(m, t.lane, [&](int dof, int n, auto tiny) {
+    const float* const Mb = M + dof * nv + dof;
+    float* const Lb = L + dof * nv + dof;
+    if constexpr (decltype(tiny)::value) {
+      TinyBlock T;
+      T.load(n, [&](int r, int c) { return Mb[r * nv + c]; });
+      T.factor(n);
+#pragma unroll
+      for (int r = 0; r < kTinyMax; r++)
+#pragma unroll
+        for (int c = 0; c < kTinyMax; c++)
+          if (r < n && c < n) Lb[r * nv + c] = c <= r ? T.a[T.at(r, c)] : 0.0f;
+    } else if (n <= kTriMax) {
       tri_load(lds, n, t.lane, [&](int r, int c) { return Mb[r * nv + c]; });
-      chol_tri(lds, n, t.lane);
-      tri_store(lds, n, L + dof * nv + dof, nv, t.lane);
+      chol_tri_block(lds, n, t.lane);
+      tri_store(lds, n, Lb, nv, t.lane);
       sync();
-      return;
+    } else {
+      for (int p = t.lane; p < n * n; p += TEAM) lds[p] = Mb[p / n * nv + p % n];
+      sync();
+      chol_lds(lds, n, n, m, t);
+      for (int p = t.lane; p < n * n; p += TEAM) Lb[p / n * nv + p % n] = lds[p];
+      sync();
     }
-    for (int p = t.lane; p < n * n; p += TEAM) lds[p] = M[(dof + p / n) * nv + dof + p % n];
-    sync();
-    chol_lds(lds, n, n, m, t);
-    for (int p = t.lane; p < n * n; p += TEAM) L[(dof + p / n) * nv + dof + p % n] = lds[p];
-    sync();
   });
 }
 
@@ -811,25 +956,10 @@ MJH_DEV void solve_blocks(const mjhModel& m, const float* L, float* x, const flo
                           const Team<TEAM>& t) {
   if constexpr (TEAM == kRegTeam) {
     reg_solve_blocks(m, L, x, y, lds, t);
-    return;
+  } else {
+    solve_tree_blocks(m, lds, t, true, L, [](float&, int) {}, [&](int i) { return y[i]; },
+                      [&](int i, float v) { x[i] = v; });
   }
-  const int nv = m.nv;
-  for_each_tree_block(m, [&](int dof, int n) {
-    if (TEAM == 64 && n <= kTriMax) {
-      const float* const Lb = L + dof * nv + dof;
-      tri_solve(lds, n, t.lane, true, [&](int r, int c) { return Lb[r * nv + c]; }, [](float&, int) {},
-                [&](int i) { return y[dof + i]; }, [&](int i, float v) { x[dof + i] = v; });
-      return;
-    }
-    float* Ls = lds;
-    float* xs = lds + n * n;
-    for (int p = t.lane; p < n * n; p += TEAM) Ls[p] = L[(dof + p / n) * nv + dof + p % n];
-    for (int p = t.lane; p < n; p += TEAM) xs[p] = y[dof + p];
-    sync();
-    cho_solve_lds(Ls, n, n, xs, t);
-    for (int p = t.lane; p < n; p += TEAM) x[dof + p] = xs[p];
-    sync();
-  });
 }
 
 // smooth.py:383-395 factor_m: the dense Cholesky factor qLDd of qMd, and

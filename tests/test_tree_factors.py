@@ -1,8 +1,8 @@
 """Mass-matrix factors on 64-lane teams: the packed blocks (one row a lane, two
-rows, the largest packed and the first that is not) and the sparse L'DL factor
-(its look-up table in LDS, also on 32-lane teams, more ancestors than a pass
-takes, and a matrix too large for the table), against float32 backward error
-bounds: |M x - b| <= g |L| |L'| |x| and |M - L' D L| <= g |L'| |D| |L|, with
+rows, the largest packed and the first that is not), small blocks, and the
+sparse L'DL factor (its look-up table in LDS, also on 32-lane teams, more
+ancestors than a pass takes, and a matrix too large for the table), against
+float32 backward error bounds: |M x - b| <= g |L| |L'| |x| and |M - L' D L| <= g |L'| |D| |L|, with
 g = 4 (3 n + 4) eps and 4 (n + 4) eps (the textbook constants times 4)."""
 import numpy as np
 import pytest
@@ -10,7 +10,7 @@ import torch
 
 import helpers
 import mjx_warp_amd as mjw
-from mjx_warp_amd import models
+from mjx_warp_amd import mjcf, models
 
 pytestmark = pytest.mark.gpu
 EPS = np.finfo(np.float32).eps
@@ -35,6 +35,40 @@ def test_packed_blocks(nv):
     H, y = M[w].astype(np.float64), x[w].cpu().numpy().astype(np.float64)
     L = np.abs(np.linalg.cholesky(H))
     assert np.all(np.abs(H @ y - b[w]) <= 4 * (3 * nv + 4) * EPS * (L @ (L.T @ np.abs(y))))
+
+
+def _chains(n, trees):
+  link = lambda k: ('<body><joint axis="0 1 0"/><geom type="capsule" fromto="0 0 0 0 0 -0.1" size="0.02"/>'
+                    + (link(k - 1) if k > 1 else "") + "</body>")
+  return mjcf.from_xml_string('<mujoco><option jacobian="dense"/><worldbody>' + trees * link(n) + "</worldbody></mujoco>")
+
+
+# a tree per lane from one dof to the most it takes (more trees than lanes
+# too), then packed: both sides of each change of panel width, several panels
+@pytest.mark.parametrize("n,trees", [(1, 65), (2, 17), (5, 7), (6, 70), (7, 5), (8, 5), (9, 4), (12, 3), (13, 3), (17, 2)])
+def test_small_blocks(n, trees):
+  nv = n * trees
+  mjm = _chains(n, trees)
+  assert mjm.nv == nv > 32
+  m = mjw.put_model(mjm)
+  d = mjw.make_data(mjm, nworld=2, nconmax=16, njmax=16)
+  rng = np.random.default_rng(n)
+  M = np.zeros((2, nv, nv), np.float32)
+  for k in range(0, nv, n):
+    A = rng.normal(size=(2, n, n))
+    M[:, k:k + n, k:k + n] = A @ A.transpose(0, 2, 1) + n * np.eye(n)
+  b = rng.normal(size=(2, nv)).astype(np.float32)
+  helpers.set_field(d, "qM", M)
+  mjw.factor_m(m, d)
+  x = torch.zeros(2, nv, device="cuda")
+  mjw.solve_m(m, d, x, torch.as_tensor(b, device="cuda"))
+  torch.cuda.synchronize()
+  F = helpers.data_numpy(d, "qLD").astype(np.float64)
+  for w in range(2):
+    H, y = M[w].astype(np.float64), x[w].cpu().numpy().astype(np.float64)
+    L = np.abs(np.linalg.cholesky(H))
+    assert np.all(np.abs(H - F[w] @ F[w].T) <= 4 * (n + 4) * EPS * (L @ L.T))
+    assert np.all(np.abs(H @ y - b[w]) <= 4 * (3 * n + 4) * EPS * (L @ (L.T @ np.abs(y))))
 
 
 @pytest.mark.parametrize("nv", [2, 17, 32, 33, 60, 126, 128])
