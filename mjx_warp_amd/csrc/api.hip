@@ -286,6 +286,7 @@ int lds_tail(const mjhModel& m, bool wide) {
 int lds_sap(const mjhModel& m) { return lds_sap_words(m.ngeom); }
 
 size_t lds_cap();
+int cu_count();
 bool reg_path(const mjhModel& m);
 int lds_forward(const mjhModel& m, bool reg);
 constexpr int kLdsRowsMin = 256, kLdsRowsMax = 1024;
@@ -420,21 +421,34 @@ int lds_solve_reg(const mjhModel& m, const Tune& t) {
   return ((a > b ? a : b) + 3) & ~3;
 }
 int lds_solve_reg(const mjhModel& m) { return lds_solve_reg(m, tune_for(m)); }
-// The big-world launch stages as many Jacobian rows as two worlds hold in a
-// quarter of a CU's LDS (40 KiB; 164 rows at nv 27), so that every SIMD gets
-// a wavefront.
-Tune tune_tail_reg(const mjhModel& m, Tune t) {
-  const int nvc = reg_nvc(m.nv);
-  const int fit = ((int)(lds_cap() / sizeof(float)) / 8 - lds_reg_floats(0, nvc, kRegSets)) / reg_row_stride(nvc) + nvc;
+// The big-world launch stages as many Jacobian rows as its LDS holds; those past
+// it are read from global memory, several times slower.  Two workgroups (of two
+// worlds) per CU stage 253 rows or more (in 64 KiB, which a launch has without
+// asking; 243 rows in 80 KiB at nv 29 to 32), four 164 at nv 27 and let every
+// SIMD have a wavefront.  So two while all workgroups are resident at once
+// anyway, else four; at nv 29 to 32, where four would stage only 101 rows, three
+// (145 rows), and two while three would leave a second round nearly empty.
+// Fused steps in us with two / three / four: 28-link chains with 202 rows, 1024
+// worlds 2390 / 2470 / 3020, 8192 15960 / 12100 / 13690; 32-link chains with 233
+// rows, 2048 worlds 4670 / 7010 / 6270, 8192 18100 / 20440 / 24990; lying
+// humanoids (nv 27, up to 140 rows), 8192 worlds 1570 / 1360 / 1270.
+// nworld: the launch's worlds, or 0 when it takes several groups'.
+constexpr int kLdsPiece = 1280;  // bytes; more than a whole number of pieces takes the next one
+Tune tune_tail_reg(const mjhModel& m, Tune t, int nworld) {
+  const int nvc = reg_nvc(m.nv), wgs = nworld / 2 + nworld % 2, cus = cu_count();
+  const int per_cu = nworld == 0 ? 4 : wgs <= 2 * cus ? 2 : nvc <= 28 ? 4 : wgs <= 4 * cus ? 2 : 3;
+  size_t bytes = lds_cap() / per_cu / kLdsPiece * kLdsPiece;
+  if (nvc <= 28 && bytes > 65536) bytes = 65536;
+  const int room = (int)(bytes / (2 * sizeof(float)));
+  const int fit = (room - lds_reg_floats(0, nvc, kRegSets)) / reg_row_stride(nvc) + nvc;
   t.rj = fit < kRegRows ? fit : kRegRows;
   return t;
 }
-Tune tune_tail_reg(const mjhModel& m) { return tune_tail_reg(m, tune_for(m)); }
+Tune tune_tail_reg(const mjhModel& m, int nworld) { return tune_tail_reg(m, tune_for(m), nworld); }
 int lds_tail_reg(const mjhModel& m, const Tune& tail) {
   const int a = lds_reg_floats(tail.rj, reg_nvc(m.nv), kRegSets), b = lds_linalg(m);
   return ((a > b ? a : b) + 3) & ~3;
 }
-int lds_tail_reg(const mjhModel& m) { return lds_tail_reg(m, tune_tail_reg(m)); }
 
 // A second stream per device and host thread for work that may run beside
 // the caller's stream (default priority; ordered against it with events).
@@ -491,25 +505,33 @@ int check_hip(hipError_t e, const char* what) {
 }
 
 // LDS bytes one workgroup may take on the current device (160 KiB on
-// gfx950), read once per device.
-size_t lds_cap() {
+// gfx950) and its CUs, read once per device.
+struct DeviceLimits {
+  size_t lds = 65536;
+  int cus = 256;
+};
+DeviceLimits device_limits() {
   static std::mutex mu;
-  static std::map<int, size_t> per_device;
+  static std::map<int, DeviceLimits> per_device;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
     (void)hipGetLastError();
-    return 65536;
+    return DeviceLimits{};
   }
   std::lock_guard<std::mutex> lock(mu);
   auto it = per_device.find(dev);
   if (it != per_device.end()) return it->second;
   int v = 0;
-  size_t cap = 65536;
-  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 0) cap = v;
+  DeviceLimits l;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 0) l.lds = v;
   else (void)hipGetLastError();
-  per_device[dev] = cap;
-  return cap;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) l.cus = v;
+  else (void)hipGetLastError();
+  per_device[dev] = l;
+  return l;
 }
+size_t lds_cap() { return device_limits().lds; }
+int cu_count() { return device_limits().cus; }
 // A launch of `kernel` with `bytes` of dynamic LDS: above 64 KiB the kernel
 // is allowed that much first.
 int allow_lds(const void* kernel, size_t bytes, const char* name) {
@@ -605,11 +627,11 @@ int do_solve(const mjhModel& m, const mjhData& d, hipStream_t s) {
   if (reg_path(m) && d.step_desc && d.nworld > 0) {
     TRY(solve_reg_desc(m, d, s));
   } else if (reg_path(m)) {
-    const Tune tt = tune_tail_reg(m);
+    const Tune tt = tune_tail_reg(m, d.nworld);
     TRY(beside(
         s,
         [&](hipStream_t q) {
-          return launch_team<StBigWorlds<false>, kRegTeam>(m, d, q, lds_tail_reg(m), "solve_big_worlds", &tt);
+          return launch_team<StBigWorlds<false>, kRegTeam>(m, d, q, lds_tail_reg(m, tt), "solve_big_worlds", &tt);
         },
         [&](hipStream_t q) { return launch_team<StSolveTeam, kRegTeam>(m, d, q, lds_solve_reg(m), "solve"); }));
   } else {
@@ -668,11 +690,11 @@ int do_step_fused(const mjhModel& m, const mjhData& d, hipStream_t s) {
     Tune tf = tune_for(m);
     tf.resident = 0;
     TRY((launch_team<StFusedForward, kRegTeam>(m, d, s, lds_forward_reg(m), "step_fused_forward", &tf)));
-    const Tune tt = tune_tail_reg(m);
+    const Tune tt = tune_tail_reg(m, d.nworld);
     TRY(beside(
         s,
         [&](hipStream_t q) {
-          return launch_team<StBigWorlds<true>, kRegTeam>(m, d, q, lds_tail_reg(m), "step_big_worlds", &tt);
+          return launch_team<StBigWorlds<true>, kRegTeam>(m, d, q, lds_tail_reg(m, tt), "step_big_worlds", &tt);
         },
         [&](hipStream_t q) {
           return launch_team<StFusedSolveIntegrate, kRegTeam>(m, d, q, lds_solve_reg(m), "step_fused_solve");
@@ -805,18 +827,19 @@ GroupDesc single_desc(const mjhModel& m, const mjhData& d) {
   g.d = d;
   g.first_block = 0;
   g.tune[0] = tune_for(m);
-  g.tune[1] = reg_path(m) ? tune_tail_reg(m) : g.tune[0];
+  g.tune[1] = reg_path(m) ? tune_tail_reg(m, d.nworld) : g.tune[0];
   return g;
 }
 
 // The 32-lane solve launches of the plain step (mjh_solve) through the
 // group kernels, as the fused step does; counters are left alone.
 int solve_reg_desc(const mjhModel& m, const mjhData& d, hipStream_t s) {
-  const int l_solve = lds_solve_reg(m), l_big = lds_tail_reg(m);
+  const GroupDesc g = single_desc(m, d);
+  const int l_solve = lds_solve_reg(m), l_big = lds_tail_reg(m, g.tune[1]);
   if ((size_t)max_of(2 * l_solve, 2 * l_big) * sizeof(float) > lds_cap())
     return fail(MJH_ERR_CAPACITY, "solve: model too large for the dense LDS kernels (nv = " + std::to_string(m.nv) + ")");
   GroupDesc* dev = reinterpret_cast<GroupDesc*>((int32_t*)d.step_desc);
-  hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(256), 0, s, single_desc(m, d), dev, 0);
+  hipLaunchKernelGGL(k_write_desc, dim3(1), dim3(256), 0, s, g, dev, 0);
   TRY(check_launch("solve: description"));
   GroupTable t32;
   t32.dev = dev;
@@ -828,15 +851,10 @@ int solve_reg_desc(const mjhModel& m, const mjhData& d, hipStream_t s) {
 }
 
 int do_step_fused_desc(const mjhModel& m, const mjhData& d, hipStream_t s) {
-  GroupDesc g{};
-  g.m = m;
-  g.d = d;
-  g.first_block = 0;
-  g.tune[0] = tune_for(m);
-  g.tune[1] = reg_path(m) ? tune_tail_reg(m) : g.tune[0];
+  const GroupDesc g = single_desc(m, d);
   GroupDesc* dev = reinterpret_cast<GroupDesc*>((int32_t*)d.step_desc);
   const bool reg = reg_path(m);
-  const int l_fwd = lds_forward_reg(m), l_solve = lds_solve_reg(m), l_big = lds_tail_reg(m), l_step = lds_step(m),
+  const int l_fwd = lds_forward_reg(m), l_solve = lds_solve_reg(m), l_big = reg ? lds_tail_reg(m, g.tune[1]) : 0, l_step = lds_step(m),
             l_tail = lds_tail(m, g.tune[0]), l_fwd64 = max_of(lds_forward(m, false), lds_linalg(m)),
             l_solve64 = lds_solve(m, g.tune[0]);
   const size_t need = reg ? (size_t)max_of(max_of(2 * l_fwd, 2 * l_solve), max_of(2 * l_big, l_tail))
@@ -889,7 +907,7 @@ int choose(int i, const mjhModel& m, const mjhGroupTune* o, Choice* c) {
   if (o && o->rj >= 0) t.rj = o->rj;
   if (t.rj > t.rmax) t.rj = t.rmax;
   c->tune[0] = t;
-  c->tune[1] = c->reg ? tune_tail_reg(m, t) : t;
+  c->tune[1] = c->reg ? tune_tail_reg(m, t, 0) : t;
   return MJH_OK;
 }
 
