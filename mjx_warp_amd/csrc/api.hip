@@ -288,7 +288,7 @@ int lds_sap(const mjhModel& m) { return lds_sap_words(m.ngeom); }
 size_t lds_cap();
 int cu_count();
 bool reg_path(const mjhModel& m);
-int lds_forward(const mjhModel& m, bool reg);
+int lds_forward(const mjhModel& m, bool reg, bool resident);
 constexpr int kLdsRowsMin = 256, kLdsRowsMax = 1024;
 
 // Row capacity of the LDS solver (rows of one world) and how many of them
@@ -332,7 +332,7 @@ Tune tune_for(const mjhModel& m, bool reg) {
       if (std::strcmp(e, "0") == 0 && fits) t.hess = kHessSquare;
     }
     int base = lds_solver_floats(m.nv, 0, t.rj, t.hess);
-    const int fwd = lds_forward(m, false);
+    const int fwd = lds_forward(m, false, true);
     if (fwd > base) base = fwd;
     if (base + 8 * kLdsRowsMin <= cap) {
       const int per_cu = cap / (base + 8 * kLdsRowsMin);
@@ -374,8 +374,8 @@ int lds_vel(const mjhModel& m) { return lds_velocity_floats(m.nbody); }
 int lds_broadphase(const mjhModel& m) { return m.ngeom > 100 ? lds_sap(m) : kNxnWords * m.ngeom; }
 int lds_con(bool reg) { return reg ? lds_constraint_floats<kRegTeam>() : lds_constraint_floats<kTeam>(); }
 // every forward stage of the fused forward launch, on 32-lane (reg) or
-// 64-lane teams
-int lds_forward(const mjhModel& m, bool reg) {
+// 64-lane teams; resident: the launch has the resident form too
+int lds_forward(const mjhModel& m, bool reg, bool resident) {
   int a = lds_kin(m);
   const int b = lds_crb(m, reg), c = lds_vel(m), g = lds_broadphase(m), k = lds_con(reg);
   a = a > b ? a : b;
@@ -383,13 +383,12 @@ int lds_forward(const mjhModel& m, bool reg) {
   a = a > k ? a : k;
   a = a > g ? a : g;
   const int team = reg ? kRegTeam : kTeam;
-  const int r = fwd_resident(m, team, (int)(lds_cap() / sizeof(float))) ? fwd_lds(m, team).total : 0;
+  const int r = resident && fwd_resident(m, team, (int)(lds_cap() / sizeof(float))) ? fwd_lds(m, team).total : 0;
   return a > r ? a : r;
 }
-int lds_forward(const mjhModel& m) { return lds_forward(m, reg_path(m)); }
 // the 64-lane fused step (forward, LDS solver, integrator in one launch)
 int lds_step(const mjhModel& m, const Tune& t) {
-  const int a = lds_solve(m, t), b = lds_forward(m, false);
+  const int a = lds_solve(m, t), b = lds_forward(m, false, false);
   return a > b ? a : b;
 }
 int lds_step(const mjhModel& m) { return lds_step(m, tune_for(m, false)); }
@@ -581,7 +580,7 @@ int launch_team(const mjhModel& m, const mjhData& d, hipStream_t s, int ldsw, co
 // at its start) is 16-byte aligned.
 int reg_stride(int ldsw) { return ((ldsw > kRegLdsMin ? ldsw : kRegLdsMin) + 3) & ~3; }
 // the fused forward launch of 32-lane teams
-int lds_forward_reg(const mjhModel& m) { return reg_stride(lds_forward(m)); }
+int lds_forward_reg(const mjhModel& m, bool resident) { return reg_stride(lds_forward(m, true, resident)); }
 
 // A stage on the model's team size: 32-lane teams (two worlds per
 // wavefront) when the register path applies, else 64-lane teams.
@@ -686,10 +685,10 @@ int do_step_fused(const mjhModel& m, const mjhData& d, hipStream_t s) {
   if (d.step_desc && d.nworld > 0) return do_step_fused_desc(m, d, s);
   TRY(reset(d, s, (m.opt.disableflags & mjhDSBL_CONSTRAINT) ? 1 : 3));
   if (reg_path(m)) {
-    // (the resident form reads the model too widely for a kernel argument)
-    Tune tf = tune_for(m);
-    tf.resident = 0;
-    TRY((launch_team<StFusedForward, kRegTeam>(m, d, s, lds_forward_reg(m), "step_fused_forward", &tf)));
+    // (the resident form reads the model too widely for a kernel argument:
+    // compiled in beside the stages, it alone put 1 KiB of it per lane in
+    // scratch memory, 196 to 444 us for 8192 humanoids)
+    TRY((launch_team<StStagedForward, kRegTeam>(m, d, s, lds_forward_reg(m, false), "step_fused_forward")));
     const Tune tt = tune_tail_reg(m, d.nworld);
     TRY(beside(
         s,
@@ -854,8 +853,9 @@ int do_step_fused_desc(const mjhModel& m, const mjhData& d, hipStream_t s) {
   const GroupDesc g = single_desc(m, d);
   GroupDesc* dev = reinterpret_cast<GroupDesc*>((int32_t*)d.step_desc);
   const bool reg = reg_path(m);
-  const int l_fwd = lds_forward_reg(m), l_solve = lds_solve_reg(m), l_big = reg ? lds_tail_reg(m, g.tune[1]) : 0, l_step = lds_step(m),
-            l_tail = lds_tail(m, g.tune[0]), l_fwd64 = max_of(lds_forward(m, false), lds_linalg(m)),
+  const int l_fwd = reg ? lds_forward_reg(m, true) : 0, l_solve = lds_solve_reg(m),
+            l_big = reg ? lds_tail_reg(m, g.tune[1]) : 0, l_step = lds_step(m),
+            l_tail = lds_tail(m, g.tune[0]), l_fwd64 = max_of(lds_forward(m, false, true), lds_linalg(m)),
             l_solve64 = lds_solve(m, g.tune[0]);
   const size_t need = reg ? (size_t)max_of(max_of(2 * l_fwd, 2 * l_solve), max_of(2 * l_big, l_tail))
                           : (size_t)max_of(split64() ? max_of(l_fwd64, l_solve64) : l_step, l_tail);
@@ -918,14 +918,14 @@ struct GroupLds {
 GroupLds group_lds(const mjhModel& m, const Choice& c) {
   GroupLds l;
   if (c.reg) {
-    l.fwd = reg_stride(lds_forward(m, true));
+    l.fwd = lds_forward_reg(m, true);
     l.solve = lds_solve_reg(m, c.tune[0]);
     l.big = lds_tail_reg(m, c.tune[1]);
     l.tail32 = lds_tail(m, c.tune[0]);
   } else {
     l.step = lds_step(m, c.tune[0]);
     l.tail64 = lds_tail(m, c.tune[0]);
-    l.fwd64 = max_of(lds_forward(m, false), lds_linalg(m));
+    l.fwd64 = max_of(lds_forward(m, false, true), lds_linalg(m));
     l.solve64 = lds_solve(m, c.tune[0]);
   }
   return l;

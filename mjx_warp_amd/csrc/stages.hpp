@@ -177,13 +177,9 @@ struct StFusedStep {
 // matrix: factor_m, qacc_smooth, the solver and the integrator.  The second
 // group keeps a world's matrix rows in VGPRs; one kernel holding both
 // groups would impose that register budget on the whole step.
-struct StFusedForward {
+struct StStagedForward {
   template <int T>
-  MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<T>& t, const Tune& tune) const {
-    if (tune.resident) {
-      forward_resident(m, d, l, t);
-      return;
-    }
+  MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<T>& t, const Tune&) const {
     kinematics(m, d, l, t);
     com_pos(m, d, l, t);
     crb(m, d, l, t);
@@ -194,6 +190,13 @@ struct StFusedForward {
     fwd_velocity(m, d, l, t);
     fwd_actuation(m, d, t);
     fwd_acceleration_force(m, d, t);
+  }
+};
+struct StFusedForward {
+  template <int T>
+  MJH_DEV void operator()(const mjhModel& m, const mjhData& d, float* l, const Team<T>& t, const Tune& tune) const {
+    if (tune.resident) forward_resident(m, d, l, t);
+    else StStagedForward()(m, d, l, t, tune);
   }
 };
 struct StFusedSolveIntegrate {
@@ -392,7 +395,7 @@ using StTailStep = StTail<true>;
 #define MJH_KERNELS_BIG_SOLVE(X, G) X(32, StBigWorldsSolve)
 #define MJH_KERNELS_BIG_SOLVE_G(X, G) G(32, StBigWorldsSolve, 1)
 // the fused step's launches
-#define MJH_KERNELS_FUSED_FORWARD(X, G) X(32, StFusedForward) G(32, StFusedForward, 0)
+#define MJH_KERNELS_FUSED_FORWARD(X, G) X(32, StStagedForward) G(32, StFusedForward, 0)
 #define MJH_KERNELS_FUSED_SOLVE(X, G) X(32, StFusedSolveIntegrate)
 #define MJH_KERNELS_FUSED_SOLVE_G(X, G) G(32, StFusedSolveIntegrate, 0)
 #define MJH_KERNELS_BIG_STEP(X, G) X(32, StBigWorldsStep)
