@@ -829,13 +829,14 @@ struct TinyBlock {
   }
 };
 // for_each_tree_block on a 64-lane team, the trees of at most kTinyMax dofs
-// handed out a tree per lane: f(dof, size, whether by the lane alone).
-template <class F>
+// handed out a tree per lane: f(dof, size, whether by the lane alone).  kTiny
+// unset: every tree by the team.
+template <bool kTiny = true, class F>
 MJH_DEV void for_each_sized_block(const mjhModel& m, int lane, F f) {
   for (int g = 0; g < m.nqLD_group; g++) {
     const int beg = m.qLD_tileadr[g], size = m.qLD_tilesize[g];
     const int end = (g == m.nqLD_group - 1) ? m.nqLD_tile : m.qLD_tileadr[g + 1];
-    if (size <= kTinyMax) {
+    if (kTiny && size <= kTinyMax) {
       for (int k = beg + lane; k < end; k += 64) f(m.qLD_tile[k], size, std::true_type{});
       sync();
       continue;
@@ -878,11 +879,11 @@ MJH_DEV void tiny_solve(int n, bool factored, F f, G diag, B b, X x) {
 // x = inv(A) b for every tree block of a 64-lane team's world: A global
 // [nv, nv] (factored: the factor's blocks), its diagonal's gain diag(entry, i),
 // b(i) and x(i, value) by dof; lds: n n + n floats of the largest block.
-template <class G, class B, class X>
+template <bool kTiny = true, class G, class B, class X>
 MJH_DEV void solve_tree_blocks(const mjhModel& m, float* lds, const Team<64>& t, bool factored, const float* A, G diag,
                                B b, X x) {
   const int nv = m.nv;
-  for_each_sized_block(m, t.lane, [&](int dof, int n, auto tiny) {
+  for_each_sized_block<kTiny>(m, t.lane, [&](int dof, int n, auto tiny) {
     const float* const Ab = A + dof * nv + dof;
     auto Af = [&](int r, int c) { return Ab[r * nv + c]; };
     auto dg = [&](float& v, int i) { diag(v, dof + i); };
@@ -951,13 +952,13 @@ MJH_DEV void factor_blocks(const mjhModel& m, const float* M, float* L, float* l
 
 // x = inv(M) y with M = L L' given by its tree blocks (smooth.py:654-681).
 // x may alias y.  lds needs nv*nv + nv floats.
-template <int TEAM>
+template <bool kTiny = true, int TEAM>
 MJH_DEV void solve_blocks(const mjhModel& m, const float* L, float* x, const float* y, float* lds,
                           const Team<TEAM>& t) {
   if constexpr (TEAM == kRegTeam) {
     reg_solve_blocks(m, L, x, y, lds, t);
   } else {
-    solve_tree_blocks(m, lds, t, true, L, [](float&, int) {}, [&](int i) { return y[i]; },
+    solve_tree_blocks<kTiny>(m, lds, t, true, L, [](float&, int) {}, [&](int i) { return y[i]; },
                       [&](int i, float v) { x[i] = v; });
   }
 }

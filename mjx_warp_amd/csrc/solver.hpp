@@ -87,7 +87,9 @@ struct SolverWorld {
     if (t.lane == 0) d.efc_grad_dot[w] = gd;
     sync();
     if (m.opt.solver == mjhSOL_CG) {
-      solve_blocks(m, d.qLDd + (size_t)w * nv * nv, Mgrad, grad, lds, t);
+      // no trees by the lane: their registers would be the whole tail launch's,
+      // which mostly runs the LDS solver (chains of 64 links: 15.6 to 17.7 ms)
+      solve_blocks<false>(m, d.qLDd + (size_t)w * nv * nv, Mgrad, grad, lds, t);
     } else {
       float* H = wide ? d.efc_h + (size_t)w * nv * nv : lds;
       float* x = wide ? lds : lds + nv * nv;
