@@ -691,57 +691,90 @@ MJH_DEV void chol_tri_block(float* A, int n, int lane) {
 // y / l given 1 / l: the quotient rounded from its residual, as a division ends,
 // without the scaling and the reciprocal that start one (a division is eleven
 // dependent instructions, and the solves below are a chain of 2 n of them).
-// div_fixup settles zeros, infinities and NaN.
+// The residual has to be exact and the reciprocal normal: the quotient is the
+// division's for l in [2^-60, 2^60], y zero or past 2^-100 and a quotient that
+// is zero or in [2^-100, 2^126].  (Past that a subnormal l has no reciprocal, a
+// small y loses the residual's low bits, and a quotient that overflows gives
+// NaN.)  A quotient q was one of these if it is past div_by_least(l, 1 / l), and
+// with it q l, which is y's size; zero may also stand for one of at most half
+// the smallest subnormal.
 MJH_DEV float div_by(float y, float l, float inv) {
   const float q = y * inv;
-  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-l, q, y), inv, q), l, y);
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-l, q, y), inv, q), l, y);  // the sign of zero
 }
+MJH_DEV float div_by_least(float l, float inv) {
+  return l >= 0x1p-60f && l <= 0x1p60f ? fmaxf(0x1p-100f, 0x1p-99f * inv) : __int_as_float(0x7f800000);
+}
+MJH_DEV bool div_by_held(float q, float least) { return q == 0.0f || (fabsf(q) >= least && fabsf(q) <= 0x1p126f); }
 
 // x = inv(L L') x for the packed factor, x one entry per lane and set (lanes
 // l and l + 64); each entry gets the operations of cho_solve_wave in its
 // order.  The rows' words do not depend on the chain and are loaded ahead.
-MJH_DEV void cho_solve_tri(const float* A, int n, float* x0, float* x1, int lane) {
+// kFast: divisions by div_by; returns whether all of them were in its range.
+// kTwo unset: n <= 64, no second set.
+template <bool kFast, bool kTwo>
+MJH_DEV bool cho_solve_tri_pass(const float* A, int n, float* x0, float* x1, int lane) {
   const int i1 = lane + 64;
-  const bool own0 = lane < n, own1 = i1 < n;
+  const bool own0 = lane < n, own1 = kTwo && i1 < n;
   const float* const r0 = A + tri_row(own0 ? lane : 0);
   const float* const r1 = A + tri_row(own1 ? i1 : 0);
   const float l0 = own0 ? r0[lane] : 1.0f, l1 = own1 ? r1[i1] : 1.0f;
   const float v0 = 1.0f / l0, v1 = 1.0f / l1;
   float y0 = own0 ? *x0 : 0.0f, y1 = own1 ? *x1 : 0.0f;
-  const int c64 = n < 64 ? n : 64;
-#pragma unroll 8
+  auto quot = [&](float y, float l, float inv) { return kFast ? div_by(y, l, inv) : y / l; };
+  const float least0 = div_by_least(l0, v0), least1 = div_by_least(l1, v1);
+  auto in_range = [&] { return div_by_held(y0, least0) && (!kTwo || div_by_held(y1, least1)); };
+  const int c64 = !kTwo || n < 64 ? n : 64;
+#pragma unroll (kFast ? 8 : 1)
   for (int k = 0; k < c64; k++) {
     const float a0 = lane > k && own0 ? r0[k] : 0.0f, a1 = own1 ? r1[k] : 0.0f;
-    const float yk = lane_value(div_by(y0, l0, v0), k);
+    const float yk = lane_value(quot(y0, l0, v0), k);
     if (lane == k) y0 = yk;
     else if (lane > k) y0 = fmaf(-a0, yk, y0);
-    y1 = fmaf(-a1, yk, y1);
+    if (kTwo) y1 = fmaf(-a1, yk, y1);
   }
-#pragma unroll 8
-  for (int k = 64; k < n; k++) {
+#pragma unroll (kFast ? 8 : 1)
+  for (int k = 64; kTwo && k < n; k++) {
     const float a1 = i1 > k && own1 ? r1[k] : 0.0f;
-    const float yk = lane_value(div_by(y1, l1, v1), k - 64);
+    const float yk = lane_value(quot(y1, l1, v1), k - 64);
     if (i1 == k) y1 = yk;
     else if (i1 > k) y1 = fmaf(-a1, yk, y1);
   }
-#pragma unroll 8
-  for (int k = n - 1; k >= 64; k--) {
+  const bool ok = in_range();
+#pragma unroll (kFast ? 8 : 1)
+  for (int k = n - 1; kTwo && k >= 64; k--) {
     const float* const row = A + tri_row(k);
     const float a0 = row[lane], a1 = i1 < k ? row[i1] : 0.0f;
-    const float xk = lane_value(div_by(y1, l1, v1), k - 64);
+    const float xk = lane_value(quot(y1, l1, v1), k - 64);
     if (i1 == k) y1 = xk;
     else if (i1 < k) y1 = fmaf(-a1, xk, y1);
     y0 = fmaf(-a0, xk, y0);
   }
-#pragma unroll 8
+#pragma unroll (kFast ? 8 : 1)
   for (int k = c64 - 1; k >= 0; k--) {
     const float a0 = lane < k ? A[tri_row(k) + lane] : 0.0f;
-    const float xk = lane_value(div_by(y0, l0, v0), k);
+    const float xk = lane_value(quot(y0, l0, v0), k);
     if (lane == k) y0 = xk;
     else if (lane < k) y0 = fmaf(-a0, xk, y0);
   }
   *x0 = y0;
   *x1 = y1;
+  return __all(ok && in_range());
+}
+template <bool kTwo>
+MJH_DEV void cho_solve_tri(const float* A, int n, float* x0, float* x1, int lane) {
+  const float b0 = *x0, b1 = *x1;
+  if (cho_solve_tri_pass<true, kTwo>(A, n, x0, x1, lane)) return;
+  // a NaN in L's diagonal or in b makes all of the solution NaN either way
+  auto nan = [&](int i, float b) { return i < n && (A[tri_row(i) + i] != A[tri_row(i) + i] || b != b); };
+  if (__any(nan(lane, b0) || (kTwo && nan(lane + 64, b1)))) return;
+  *x0 = b0;
+  *x1 = b1;
+  cho_solve_tri_pass<false, kTwo>(A, n, x0, x1, lane);
+}
+MJH_DEV void cho_solve_tri(const float* A, int n, float* x0, float* x1, int lane) {
+  if (n <= 64) cho_solve_tri<false>(A, n, x0, x1, lane);
+  else cho_solve_tri<true>(A, n, x0, x1, lane);
 }
 
 // The lower triangle f(row, column) into packed A, and a factor from packed A

@@ -71,6 +71,41 @@ def test_small_blocks(n, trees):
     assert np.all(np.abs(H @ y - b[w]) <= 4 * (3 * n + 4) * EPS * (L @ (L.T @ np.abs(y))))
 
 
+@pytest.mark.parametrize("nv", [40, 100])
+def test_solve_divides_at_the_ends_of_the_range(nv):
+  """A diagonal factor: every entry is two divisions, to the bit, for divisors
+  and dividends down to subnormal and up to the largest, and a quotient that
+  overflows (which the zeros off the diagonal then carry on as NaN)."""
+  mjm = models.chain(nv)
+  m = mjw.put_model(mjm)
+  rng = np.random.default_rng(nv)
+  f32 = np.float32
+  mant = lambda: rng.uniform(1, 2, nv).astype(f32)
+  ones = np.ones(nv, f32)
+  scale = lambda e: (mant() * f32(2.0) ** np.asarray(e, f32)).astype(f32)
+  sub = rng.integers(1, 1 << 23, nv).astype(np.uint32).view(f32)
+  cases = [(mant(), scale(-rng.integers(100, 126, nv))), (mant(), sub), (scale(-rng.integers(100, 126, nv)), scale(rng.integers(-126, -100, nv))),
+           (sub, sub), (scale(rng.integers(100, 127, nv)), scale(rng.integers(60, 127, nv))), (mant(), np.where(np.arange(nv) % 3 == 0, f32(0), mant())),
+           (scale(rng.integers(-20, 20, nv)), scale(rng.integers(-60, 60, nv))), (ones * f32(0.01), np.where(np.arange(nv) == nv - 2, f32(3e38), mant()))]
+  d = mjw.make_data(mjm, nworld=len(cases), nconmax=16, njmax=16)
+  L = np.stack([np.diag(l) for l, _ in cases])
+  helpers.set_field(d, "qLDd" if m.opt.is_sparse else "qLD", L)
+  y = torch.as_tensor(np.stack([y for _, y in cases]), device="cuda")
+  x = torch.zeros(len(cases), nv, device="cuda")
+  mjw.solve_m(m, d, x, y)
+  torch.cuda.synchronize()
+  with np.errstate(all="ignore"):
+    for w, (l, b) in enumerate(cases):
+      q = (b / l).astype(f32)
+      bad = np.flatnonzero(~np.isfinite(q))
+      if bad.size:
+        q[bad[0] + 1:] = np.nan
+      want = (q / l).astype(f32)
+      if np.any(~np.isfinite(want)):
+        want[: np.flatnonzero(~np.isfinite(want))[-1]] = np.nan
+      assert np.array_equal(x[w].cpu().numpy(), want, equal_nan=True), w
+
+
 @pytest.mark.parametrize("nv", [2, 17, 32, 33, 60, 126, 128])
 def test_sparse_factor(nv):
   mjm = models.chain(nv)
