@@ -76,3 +76,23 @@ def test_fused_step_pairs_match_oracle(ngeom, movers):
   oracle.run("kinematics", hm, hd)
   oracle.run("collision", hm, hd)
   _same_pairs(d, hd, 3)
+
+
+# one wavefront a world, two worlds (nv 30) or one (nv 48) in it: the smallest
+# model, more candidates than a lane has bits for (64 chunks of 32 or 64), the
+# last with staged filter ints and the first without
+@pytest.mark.parametrize("ngeom,spread", [(101, 0.5), (400, 0.3), (1024, 1.0), (1025, 1.0)])
+@pytest.mark.parametrize("movers", [5, 8])
+def test_one_wavefront_pairs_match_oracle(ngeom, spread, movers):
+  mjm = _scene(ngeom, movers, spread)
+  assert mjm.nv == 6 * movers
+  mjm.opt.disableflags |= int(mjw.DisableBit.CONSTRAINT)
+  m, d, hm, hd = _inputs(mjm, 3, 32768)
+  mjw.step_fused(m, d)
+  torch.cuda.synchronize()
+  oracle.run("kinematics", hm, hd)
+  oracle.run("collision", hm, hd)
+  assert not np.any(hd["overflow"])
+  _same_pairs(d, hd, 3)
+  if ngeom == 400:
+    assert helpers.data_numpy(d, "sap_cumulative_sum").reshape(3, -1)[:, ngeom - 1].min() > 64 * 64
