@@ -1,7 +1,8 @@
 """The big-world solve at the row counts where its work changes hands: the last
 rows staged in LDS and the first read from global memory, for the launches of
 few, some and many worlds, and the most rows it takes -- the same bits wherever a
-row is read from, against the optimum in 64 bits; and in a captured graph."""
+row is read from, against the optimum in 64 bits; in a captured graph; and on
+rows that the caller laid out, again and again on the same Data."""
 import numpy as np
 import pytest
 import torch
@@ -9,6 +10,7 @@ import torch
 import helpers
 import mjx_warp_amd as mjw
 from mjx_warp_amd import mjcf, models
+from test_big_worlds import _lying
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +96,51 @@ def test_captured(links):
     assert helpers.data_numpy(d, "world_efc").reshape(-1, 2)[:3, 1].min() > 64
     out.append((d.qpos.clone(), d.qvel.clone()))
   assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+def _lay_out(d2, d, layout, rng):
+  """d's smooth quantities and rows into d2's pool, its blocks left stale."""
+  for f in ("qM", "qLD", "qacc_smooth", "qfrc_smooth"):
+    getattr(d2, f).copy_(getattr(d, f))
+  d2.qacc_warmstart.zero_()
+  blocks = helpers.world_blocks(helpers.data_numpy(d, "world_efc"), d.nworld)
+  tag = np.concatenate([np.full(n, w) for w, (_, n) in enumerate(blocks)])
+  src = np.concatenate([np.arange(b, b + n) for b, n in blocks])
+  if layout == "interleaved":  # a random merge that keeps each world's order
+    seq = rng.permutation(tag)
+    take = np.empty(len(seq), int)
+    for w in range(d.nworld):
+      take[seq == w] = np.flatnonzero(tag == w)
+    src, tag = src[take], seq
+  n, njmax = len(src), d2.njmax
+  for f in ("J", "D", "aref", "pos", "margin"):
+    full = helpers.data_numpy(d, "efc_" + f)[src]
+    helpers.set_field(d2, "efc_" + f, np.concatenate([full, np.zeros((njmax - n,) + full.shape[1:], full.dtype)]))
+  helpers.set_field(d2, "efc_worldid", np.concatenate([tag, np.full(njmax - n, -1)]).astype(np.int32))
+  helpers.set_field(d2, "nefc", np.array([n], np.int32))
+
+
+@pytest.mark.parametrize("desc", [True, False])
+@pytest.mark.parametrize("layouts", [("blocks", "interleaved"), ("interleaved", "blocks")])
+def test_caller_laid_big_worlds(layouts, desc):
+  nworld = 5
+  mjm = models.humanoid(iterations=10, ls_iterations=20)
+  m = mjw.put_model(mjm)
+  d2 = mjw.make_data(mjm, nworld=nworld, nconmax=8, njmax=2500)
+  if not desc:
+    d2.ndesc = 0
+    d2.step_desc = torch.zeros(0, dtype=torch.int32, device="cuda")
+  rng = np.random.default_rng(len(layouts[0]))
+  for turn, layout in enumerate(layouts):  # the second turn's big worlds are others
+    d = mjw.make_data(mjm, nworld=nworld, nconmax=64 * nworld, njmax=277 * nworld)
+    helpers.set_field(d, "qpos", np.roll(_lying(mjm, nworld, 2), turn, 0))
+    mjw.forward(m, d)
+    torch.cuda.synchronize()
+    rows = helpers.data_numpy(d, "world_efc").reshape(-1, 2)[:nworld, 1]
+    assert [i for i in range(nworld) if rows[i] > 64] == ([1, 3] if turn == 0 else [2, 4]) and rows.max() <= 256
+    _lay_out(d2, d, layout, rng)
+    mjw.solve(m, d2)
+    torch.cuda.synchronize()
+    assert not np.any(helpers.data_numpy(d2, "world_flags"))
+    for f in ("qacc", "qfrc_constraint"):
+      assert torch.equal(getattr(d2, f), getattr(d, f)), (turn, f)
