@@ -72,3 +72,53 @@ def test_resident_forward_equals_stages(name, nworld):
     for f in fields:
       a, b = (helpers.gather_world_rows(get(k, prefix + f), blocks[k]) for k in range(2))
       close(a, b, prefix + f)
+
+
+def _more_bodies_than_lanes():
+  """34 bodies, 30 of them fixed, joints of three kinds: the largest such layout
+  that a 32-lane team keeps in LDS."""
+  joint = {0: '<joint axis="0 1 0" stiffness="2" damping=".1"/>', 15: '<joint type="ball"/>',
+           31: '<joint type="slide" axis="0 0 1"/>'}
+  body = lambda i: (f'<body pos=".02 0 -.05" euler="0 {3 * i} 5"><inertial pos="0 0 .01" mass=".1" diaginertia="1e-4 2e-4 3e-4"/>'
+                    + joint.get(i, "") + ('<geom size=".02"/>' if i % 15 == 0 else ""))
+  return mjcf.from_xml_string('<mujoco><option jacobian="dense"/><worldbody><geom type="plane" size="5 5 .1"/>'
+                              + "".join(body(i) for i in range(33)) + "</body>" * 33 + "</worldbody></mujoco>")
+
+
+def _heap():
+  """64-lane teams, 90 and more pairs: the pair list is emptied and begun again."""
+  ball = lambda i: f'<body pos="{.02 * (i % 4)} {.02 * (i // 4)} .05"><freejoint/><geom size=".1"/></body>'
+  return mjcf.from_xml_string('<mujoco><option jacobian="dense"/><worldbody><geom type="plane" size="5 5 .1"/>'
+                              + "".join(ball(i) for i in range(14)) + "</worldbody></mujoco>")
+
+
+@pytest.mark.parametrize("name", ["humanoid", "three", "crowd", "box", "pendula.xml", "constraints.xml", "collision.xml",
+                                  "bodies", "heap"])
+def test_resident_forward_is_the_stages_bit_for_bit(name):
+  nworld = 5
+  mjm = _more_bodies_than_lanes() if name == "bodies" else _heap() if name == "heap" else _scene(name)
+  m = mjw.put_model(mjm)
+  rng = np.random.default_rng(nworld)
+  q = np.tile(np.asarray(mjm.qpos0, np.float64), (nworld, 1)) + rng.normal(0.0, 0.05, (nworld, mjm.nq))
+  state = {"qpos": q, "qvel": rng.normal(0.0, 0.3, (nworld, mjm.nv)), "ctrl": rng.uniform(-1.0, 1.0, (nworld, mjm.nu)),
+           "xfrc_applied": rng.normal(0.0, 1.0, (nworld, mjm.nbody, 6)), "qfrc_applied": rng.normal(0.0, 1.0, (nworld, mjm.nv))}
+  out = []
+  for step in (mjw.step_fused, mjw.step):
+    d = mjw.make_data(mjm, nworld=nworld, nconmax=256 * nworld, njmax=1024 * nworld)
+    for f, v in state.items():
+      helpers.set_field(d, f, v)
+    step(m, d)
+    torch.cuda.synchronize()
+    out.append(d)
+  get = lambda k, f: helpers.data_numpy(out[k], f)
+  assert not np.any(get(0, "overflow"))
+  if name == "heap":
+    assert min(n for _, n in helpers.world_blocks(get(0, "world_pair"), nworld)) > 64
+  for f in WORLD:
+    assert np.array_equal(get(0, f), get(1, f), equal_nan=True), f
+  for fields, prefix, world in ((CONTACT, "contact_", "world_con"), (ROW, "efc_", "world_efc")):
+    blocks = [helpers.world_blocks(get(k, world), nworld) for k in range(2)]
+    assert [n for _, n in blocks[0]] == [n for _, n in blocks[1]]
+    for f in fields:
+      a, b = (helpers.gather_world_rows(get(k, prefix + f), blocks[k]) for k in range(2))
+      assert np.array_equal(a, b, equal_nan=True), prefix + f
