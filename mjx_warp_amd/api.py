@@ -224,6 +224,9 @@ def rollout(m: Model, d: Data, nstep: int, fused: bool = True):
   d.time = d.time + nstep * m.opt.timestep
 
 
+_captured = []  # the graphs of every StepGraph made, see there
+
+
 class StepGraph:
   """`nstep` consecutive steps captured once as a HIP graph and replayed.
 
@@ -235,6 +238,14 @@ class StepGraph:
   launches them on the current stream.  Replays read and write the same
   Model / Data tensors that were captured; `d.time` is advanced on the
   host by each replay, as `step` does.
+
+  The captured graph lives until the process ends, also when its StepGraph is
+  gone (some ten kilobytes per captured step; the Model and Data are released with
+  the StepGraph, which must not be replayed after that).  Destroyed graphs were
+  followed by a damaged host heap -- a dictionary that no longer found a key,
+  in a process that freed captured chain rollouts after several hundred replays
+  and captured others -- and keeping them ended it; nothing in this library's
+  code was found that explains it, so none is destroyed.
   """
 
   def __init__(self, m: Model, d: Data, nstep: int = 1, fused: bool = True):
@@ -252,6 +263,7 @@ class StepGraph:
     with torch.cuda.graph(self.graph, stream=side):
       for _ in range(self.nstep):
         _native.call(name, m, d)
+    _captured.append(self.graph)
     torch.cuda.current_stream().wait_stream(side)
 
   def replay(self):

@@ -139,3 +139,21 @@ def test_fused_step_description_path_equals_argument_path_64_lane():
   for f in ("qpos", "qvel", "qacc", "qacc_warmstart"):
     a, b = helpers.data_numpy(out[0], f), helpers.data_numpy(out[1], f)
     assert np.isfinite(a).all() and np.array_equal(a, b), (f, np.abs(a - b).max())
+
+
+def test_captured_graphs_outlive_their_step_graphs():
+  import gc
+  import weakref
+
+  mjm = models.chain(3)
+  m = mjw.put_model(mjm)
+  refs = []
+  for _ in range(2):
+    d = mjw.make_data(mjm, nworld=2, nconmax=32, njmax=128)
+    g = mjw.StepGraph(m, d)
+    g.replay()
+    torch.cuda.synchronize()
+    refs.append((weakref.ref(g.graph), weakref.ref(d)))
+    del g, d
+    gc.collect()
+  assert all(graph() is not None and data() is None for graph, data in refs)
