@@ -194,7 +194,7 @@ struct RegChol {
     gfloat* Lc = opaque(L) + (lane < nv ? lane : 0);
     wave_fence();
     if (lane < NVC) {
-#pragma unroll 7
+#pragma unroll 7  // seven or eight: the same within 1 % at 27 dofs
       for (int r = 0; r < nv; r++) rows[r * JS + lane] = Lc[r * nv];
     }
     wave_fence();
