@@ -309,8 +309,11 @@ constexpr int kLdsRowsMin = 256, kLdsRowsMax = 1024;
 // global-memory tail.  MJH_SOLVER_RMAX / MJH_SOLVER_RJ override the
 // defaults, MJH_SOLVER_WIDE=1 / 0 puts the Hessian of any 64-lane model in
 // efc_h / square in LDS (where it fits).
-Tune tune_for(const mjhModel& m, bool reg) {
+// shared: other models' groups take part in the launches.
+Tune tune_for(const mjhModel& m, bool reg, bool shared = false) {
   Tune t{64, 0, 0, 0, 0};
+  const int per_cu = !reg ? 8 : shared ? 32 : 16;  // worlds
+  t.resident = fwd_resident(m, reg ? kRegTeam : kTeam, (int)(lds_cap() / sizeof(float)) / per_cu);
   if (reg) {
     // as many Jacobian rows as leave a CU twelve workgroups (three wavefronts
     // per SIMD, what the registers allow), at least the nvc the solver's
@@ -332,7 +335,7 @@ Tune tune_for(const mjhModel& m, bool reg) {
       if (std::strcmp(e, "0") == 0 && fits) t.hess = kHessSquare;
     }
     int base = lds_solver_floats(m.nv, 0, t.rj, t.hess);
-    const int fwd = lds_forward(m, false, true);
+    const int fwd = lds_forward(m, false, t.resident);
     if (fwd > base) base = fwd;
     if (base + 8 * kLdsRowsMin <= cap) {
       const int per_cu = cap / (base + 8 * kLdsRowsMin);
@@ -352,7 +355,6 @@ Tune tune_for(const mjhModel& m, bool reg) {
   t.tail_rows = !reg && lds_solver_floats(m.nv, kLdsRowsMax, 0, t.hess) <= (int)(lds_cap() / sizeof(float))
                     ? kLdsRowsMax
                     : 0;
-  t.resident = fwd_resident(m, reg ? kRegTeam : kTeam, (int)(lds_cap() / sizeof(float)));
   return t;
 }
 Tune tune_for(const mjhModel& m) { return tune_for(m, reg_path(m)); }
@@ -374,7 +376,7 @@ int lds_vel(const mjhModel& m) { return lds_velocity_floats(m.nbody); }
 int lds_broadphase(const mjhModel& m) { return m.ngeom > 100 ? lds_sap(m) : kNxnWords * m.ngeom; }
 int lds_con(bool reg) { return reg ? lds_constraint_floats<kRegTeam>() : lds_constraint_floats<kTeam>(); }
 // every forward stage of the fused forward launch, on 32-lane (reg) or
-// 64-lane teams; resident: the launch has the resident form too
+// 64-lane teams; resident: the model takes the resident form (Tune)
 int lds_forward(const mjhModel& m, bool reg, bool resident) {
   int a = lds_kin(m);
   const int b = lds_crb(m, reg), c = lds_vel(m), g = lds_broadphase(m), k = lds_con(reg);
@@ -382,8 +384,7 @@ int lds_forward(const mjhModel& m, bool reg, bool resident) {
   a = a > c ? a : c;
   a = a > k ? a : k;
   a = a > g ? a : g;
-  const int team = reg ? kRegTeam : kTeam;
-  const int r = resident && fwd_resident(m, team, (int)(lds_cap() / sizeof(float))) ? fwd_lds(m, team).total : 0;
+  const int r = resident ? fwd_lds(m, reg ? kRegTeam : kTeam).total : 0;
   return a > r ? a : r;
 }
 // the 64-lane fused step (forward, LDS solver, integrator in one launch)
@@ -853,9 +854,9 @@ int do_step_fused_desc(const mjhModel& m, const mjhData& d, hipStream_t s) {
   const GroupDesc g = single_desc(m, d);
   GroupDesc* dev = reinterpret_cast<GroupDesc*>((int32_t*)d.step_desc);
   const bool reg = reg_path(m);
-  const int l_fwd = reg ? lds_forward_reg(m, true) : 0, l_solve = lds_solve_reg(m),
+  const int l_fwd = reg ? lds_forward_reg(m, g.tune[0].resident) : 0, l_solve = lds_solve_reg(m),
             l_big = reg ? lds_tail_reg(m, g.tune[1]) : 0, l_step = lds_step(m),
-            l_tail = lds_tail(m, g.tune[0]), l_fwd64 = max_of(lds_forward(m, false, true), lds_linalg(m)),
+            l_tail = lds_tail(m, g.tune[0]), l_fwd64 = max_of(lds_forward(m, false, g.tune[0].resident), lds_linalg(m)),
             l_solve64 = lds_solve(m, g.tune[0]);
   const size_t need = reg ? (size_t)max_of(max_of(2 * l_fwd, 2 * l_solve), max_of(2 * l_big, l_tail))
                           : (size_t)max_of(split64() ? max_of(l_fwd64, l_solve64) : l_step, l_tail);
@@ -902,7 +903,7 @@ int choose(int i, const mjhModel& m, const mjhGroupTune* o, Choice* c) {
     if (o->team == kRegTeam && m.nv > kRegNvMax) return fail(MJH_ERR_INVALID, g + "32-lane teams need nv <= 32");
     if (o->team) c->reg = o->team == kRegTeam;
   }
-  Tune t = tune_for(m, c->reg);
+  Tune t = tune_for(m, c->reg, true);
   if (o && o->rmax > 0) t.rmax = o->rmax;
   if (o && o->rj >= 0) t.rj = o->rj;
   if (t.rj > t.rmax) t.rj = t.rmax;
@@ -918,14 +919,14 @@ struct GroupLds {
 GroupLds group_lds(const mjhModel& m, const Choice& c) {
   GroupLds l;
   if (c.reg) {
-    l.fwd = lds_forward_reg(m, true);
+    l.fwd = lds_forward_reg(m, c.tune[0].resident);
     l.solve = lds_solve_reg(m, c.tune[0]);
     l.big = lds_tail_reg(m, c.tune[1]);
     l.tail32 = lds_tail(m, c.tune[0]);
   } else {
     l.step = lds_step(m, c.tune[0]);
     l.tail64 = lds_tail(m, c.tune[0]);
-    l.fwd64 = max_of(lds_forward(m, false, true), lds_linalg(m));
+    l.fwd64 = max_of(lds_forward(m, false, c.tune[0].resident), lds_linalg(m));
     l.solve64 = lds_solve(m, c.tune[0]);
   }
   return l;

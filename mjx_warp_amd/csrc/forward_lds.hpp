@@ -17,7 +17,7 @@
 // What bounds it: with 8192 worlds, four wavefronts per SIMD, the latency of
 // the dependent steps (LDS and L2) of each world; so the layout is kept to
 // 1280 floats per world at humanoid size (16 workgroups of two worlds per
-// CU).
+// CU; larger models, see fwd_resident).
 #pragma once
 
 #include "constraint.hpp"
@@ -75,13 +75,16 @@ __host__ __device__ inline FwdLds fwd_lds(const mjhModel& m, int team) {
   return fwd_lds(m.nq, m.nv, m.nbody, m.njnt, m.ngeom, m.nu, team);
 }
 // Whether the layout serves the model on teams of this size: pairs from the
-// nxn table, at most 64 bodies (a dof's subtree as one 64-bit mask) and two
-// dofs per lane, and no more LDS than 16 (32-lane teams) or 8 (64-lane)
-// workgroups per CU leave, beyond which the stage functions' smaller layouts
-// keep more wavefronts in flight.
-__host__ __device__ inline bool fwd_resident(const mjhModel& m, int team, int lds_cap_floats) {
-  return m.ngeom <= MJH_NXN_TABLE_MAX && m.nbody <= 64 && m.nv <= 2 * team &&
-         fwd_lds(m, team).total <= (team == 64 ? lds_cap_floats / 8 : lds_cap_floats / 32);
+// nxn table, at most 64 bodies (a dof's subtree as one 64-bit mask), two dofs
+// per lane and at most `limit` floats.  The limit is eight workgroups a CU (2560
+// floats on 32-lane teams, 5120 on 64-lane ones; two wavefronts a SIMD), and
+// sixteen on 32-lane teams where groups of other models share the launch and its
+// LDS.  Fused steps in us, stage functions / resident, at 1024, 8192 and 32768
+// worlds: a 20-link chain (1316 floats) 162 / 138, 289 / 299, 1021 / 759; the
+// humanoid with four more bodies (1396) 313 / 294, 534 / 532, 1746 / 1494; a
+// 32-link chain (2036) 217 / 177, 563 / 436, 1814 / 1387.
+__host__ __device__ inline bool fwd_resident(const mjhModel& m, int team, int limit) {
+  return m.ngeom <= MJH_NXN_TABLE_MAX && m.nbody <= 64 && m.nv <= 2 * team && fwd_lds(m, team).total <= limit;
 }
 
 // n consecutive words from LDS to global memory, lanes over words

@@ -74,15 +74,14 @@ def test_resident_forward_equals_stages(name, nworld):
       close(a, b, prefix + f)
 
 
-def _more_bodies_than_lanes():
-  """34 bodies, 30 of them fixed, joints of three kinds: the largest such layout
-  that a 32-lane team keeps in LDS."""
+def _more_bodies_than_lanes(n):
+  """n bodies under the world, all but three fixed, joints of three kinds."""
   joint = {0: '<joint axis="0 1 0" stiffness="2" damping=".1"/>', 15: '<joint type="ball"/>',
            31: '<joint type="slide" axis="0 0 1"/>'}
   body = lambda i: (f'<body pos=".02 0 -.05" euler="0 {3 * i} 5"><inertial pos="0 0 .01" mass=".1" diaginertia="1e-4 2e-4 3e-4"/>'
                     + joint.get(i, "") + ('<geom size=".02"/>' if i % 15 == 0 else ""))
   return mjcf.from_xml_string('<mujoco><option jacobian="dense"/><worldbody><geom type="plane" size="5 5 .1"/>'
-                              + "".join(body(i) for i in range(33)) + "</body>" * 33 + "</worldbody></mujoco>")
+                              + "".join(body(i) for i in range(n)) + "</body>" * n + "</worldbody></mujoco>")
 
 
 def _heap():
@@ -93,10 +92,12 @@ def _heap():
 
 
 @pytest.mark.parametrize("name", ["humanoid", "three", "crowd", "box", "pendula.xml", "constraints.xml", "collision.xml",
-                                  "bodies", "heap"])
+                                  "bodies33", "bodies63", "bodies64", "chain32", "heap"])
 def test_resident_forward_is_the_stages_bit_for_bit(name):
   nworld = 5
-  mjm = _more_bodies_than_lanes() if name == "bodies" else _heap() if name == "heap" else _scene(name)
+  # (63 bodies: with the world's the most that the resident form takes)
+  mjm = (_more_bodies_than_lanes(int(name[6:])) if name.startswith("bodies") else _heap() if name == "heap"
+         else models.chain(32) if name == "chain32" else _scene(name))
   m = mjw.put_model(mjm)
   rng = np.random.default_rng(nworld)
   q = np.tile(np.asarray(mjm.qpos0, np.float64), (nworld, 1)) + rng.normal(0.0, 0.05, (nworld, mjm.nq))
