@@ -15,8 +15,8 @@
 // are bank-conflict free; rows past the staged count are read from global
 // memory, where they are read-only during the solve.
 //
-// Cross-lane sums are DPP butterflies inside 16-lane rows plus one swizzle
-// across the two rows of a team; every lane of the team ends with the same
+// Cross-lane sums are DPP butterflies inside 16-lane rows plus one
+// v_permlane16_swap between the two rows of a team; every lane of the team ends with the same
 // bits, so per-world decisions (line-search bracket, done) stay uniform.
 // Vectors that every lane needs whole are broadcast through a 32-float LDS
 // buffer: LDS instructions of one wavefront execute in issue order, so a
